@@ -47,6 +47,9 @@ HIPCC_FLAGS = [
     "-Wl,-soname,libsuika_reshard.so",
     # packed-FP32 instructions stay disabled for all device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # kernel arguments arrive in scalar registers: a copy workgroup's first
+    # load does not wait for them
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-Wall",
     "-Wno-unused-function",
 ]
@@ -62,8 +65,8 @@ def hipcc_path() -> str:
 def build(verbose: bool = False, out: Path = LIB, defines=()) -> Path:
     """Compile the library (always recompiles) and return its path.
 
-    ``defines`` are extra ``NAME=VALUE`` macros (kernel tuning knobs such as
-    SR_UNROLL / SR_BLOCK) for building variants elsewhere than ``out``."""
+    ``defines`` are extra ``NAME=VALUE`` macros for building variants
+    elsewhere than ``out``."""
     out = Path(out)
     out.parent.mkdir(parents=True, exist_ok=True)
     tmp = out.with_suffix(".so.tmp")

@@ -17,24 +17,34 @@
 //     destination stride.  Regions that are contiguous on both sides are
 //     collapsed to one long row.
 //   * Items are cut into tiles of `tile_bytes` (16 KiB) source bytes; one
-//     workgroup (512 lanes = 8 wave64) processes one tile in a single pass,
+//     workgroup (1024 lanes = 16 wave64) moves one tile, 16 bytes per lane,
 //     and the grid is the tile count (or a grid-stride loop when capped).
 //     Tiles balance the work whatever the tensor sizes (8 KB norms to GB
 //     embeddings).
-//   * The tile list follows the tensor address each item starts at and is
-//     interleaved 8 ways: workgroups go to the 8 XCDs round-robin, so each XCD
-//     walks one contiguous eighth of the work and the tiles in flight come
-//     from 8 distant regions.  On the Llama2-7B share this takes the unpack
-//     from 8.5 to 7.4 ms; a single window of consecutive tiles keeps the read
-//     and write streams at a fixed distance and leaves HBM bandwidth idle.
+//   * A lane loads once, stores once and ends.  Two workgroups fill a compute
+//     unit, so 32 KiB of reads are in flight there: HBM moves a flat copy at
+//     6.7 TB/s with that, at 6.2 with twice as much (two loads per lane), and
+//     at 4.1-5.4 with waves that go on to another tile, because a load's data
+//     is waited for behind the stores issued before it.
+//   * So the way from the launch to the load is short: the kernel arguments
+//     arrive in registers, a tile's record holds the addresses of a
+//     contiguous copy, a record line is read into the die's L2 256 tiles
+//     before its workgroup starts (without that: 6.4 TB/s), and the forms of
+//     large tensors come first in a kernel of 20 KB (46 KB: 3% slower).
+//   * The tile list follows the tensor address each item starts at and is cut
+//     into 8 segments: workgroups go to the 8 XCDs round-robin, so each XCD
+//     walks one contiguous eighth of the list (and of its records) and the
+//     tiles in flight come from 8 distant regions; a single window of
+//     consecutive tiles keeps the read and write streams at a fixed distance
+//     and leaves HBM bandwidth idle.
 //     Side-by-side strided items (the column bands of one dim -1 `cat`) deal
 //     out their tiles row block by row block, so each destination row is
 //     written by adjacent tiles.
-//   * Lanes move 16-byte vectors (8/4/2/1 when a region is not 16-byte
-//     aligned), two independent loads in flight before the stores.
-//     Consecutive lanes touch consecutive 16-byte words of a row, so every
-//     wave access is a coalesced 1 KB burst.  Loads and stores are
-//     non-temporal by default: every byte is touched once.
+//   * Lanes move 16-byte vectors where addresses, strides and row widths are
+//     multiples of 16 bytes, and at any alignment in contiguous pieces and in
+//     long rows of 1- and 2-byte alignment; narrower vectors otherwise
+//     (bind_item).  Loads are non-temporal, and how stores are cached follows
+//     from whether they write whole lines (Policy).
 //   * Strided regions (row-parallel dim -1 slices) map a tile-relative byte
 //     position to (row, col) with a multiply-high division by the row width
 //     (Granlund-Montgomery invariant-integer division), computed per item
@@ -53,12 +63,13 @@
 //   * The O(tiles) work runs on the GPU at first use of a phase: prefix sums
 //     (wave64 shuffle scans, wave totals through LDS) give each peer's
 //     256-byte aligned buffer offsets and each item's first tile, and an emit
-//     kernel writes the tile table in its XCD-interleaved order.  The
+//     kernel writes the tile table.  The
 //     Llama2-7B share has 1.44 M tiles per phase; building them on the host
 //     took 0.12 s and a 35 MB upload per phase.
-//   * Item tables hold absolute addresses.  When the caller's pointers
-//     change, only the pointer table is uploaded and a bind kernel rebuilds
-//     the items from the descriptors and the device-side buffer offsets.
+//   * Tile records and items hold absolute addresses.  When the caller's
+//     pointers change, only the pointer table is uploaded and the emit kernel
+//     writes both again from the descriptors and the device-side buffer
+//     offsets.
 
 #include <hip/hip_runtime.h>
 
@@ -108,38 +119,21 @@ int dtype_size(int32_t dt) {
 
 namespace {
 
-#ifndef SR_BLOCK
-#define SR_BLOCK 512
-#endif
-#ifndef SR_UNROLL
-#define SR_UNROLL 2
-#endif
-constexpr int kBlock = SR_BLOCK;
-constexpr int kUnroll = SR_UNROLL;
-// Strided and recast paths carry two or three 64-bit offsets per vector;
-// a smaller unroll keeps the kernel's register count (and so its occupancy)
-// set by the contiguous copy path.
-#ifndef SR_UNROLL_STRIDED
-#define SR_UNROLL_STRIDED (SR_UNROLL < 4 ? SR_UNROLL : 4)
-#endif
-constexpr int kUnrollStrided = SR_UNROLL_STRIDED;
-constexpr uint32_t kDefaultTileBytes = 16384;   // one 512-lane x 2 x 16 B pass
+// A copy workgroup: 1024 lanes that each hold one 16-byte vector (or as many
+// narrower ones as make 16 bytes) of a 16 KiB tile.
+constexpr int kBlock = 1024;
+constexpr uint32_t kPassBytes = kBlock * 16;
+constexpr uint32_t kDefaultTileBytes = kPassBytes;
 constexpr uint64_t kBufAlign = 256;
-// Tile-list interleave width: the accelerator complex dies (XCDs) of an
-// MI355X, which take workgroups round-robin.
-#ifndef SR_INTERLEAVE_WAYS
-#define SR_INTERLEAVE_WAYS 8
-#endif
-constexpr uint32_t kXcds = SR_INTERLEAVE_WAYS;
+// Segments of the tile list, one per accelerator complex die (XCD) of an
+// MI355X; the dies take workgroups round-robin.
+constexpr uint32_t kXcds = 8;
 constexpr uint32_t kMaxGrid = 0xffffffffu / kBlock;    // grid work-items stay below 2^32
 // A RECAST item that writes the f32 copy and the bf16 copy moves 2.5x its
-// source bytes (a COPY item 2x); its tiles hold tile_bytes >> this many
-// source bytes, so a workgroup's pass stays near a copy tile's traffic.
-#ifndef SR_RECAST_TILE_SHIFT
-#define SR_RECAST_TILE_SHIFT 1
-#endif
-constexpr uint32_t kRecastTileShift = SR_RECAST_TILE_SHIFT;
-static_assert(kRecastTileShift <= 2, "RECAST tiles of at least tile_bytes / 4 (>= 1 KiB)");
+// source bytes (a COPY item 2x); its tiles, as plans count them, hold
+// tile_bytes >> this many source bytes.  A workgroup takes two of them: it
+// has lanes for tile_bytes.
+constexpr uint32_t kRecastTileShift = 1;
 
 // ---------------------------------------------------------------- errors
 
@@ -194,8 +188,8 @@ enum : uint32_t {
   kKindZero = 2,
 };
 
-// Item flags: bits 0-3 kind, 4-7 log2(vector bytes) (COPY/ZERO) or
-// log2(elements per lane vector) (RECAST), bit 8: RECAST also writes f32.
+// One piece bound to its objects' addresses: what its tiles read beyond
+// their own records.
 struct alignas(16) DevItem {
   uint64_t src;           // absolute address of the region origin
   uint64_t dst;
@@ -206,18 +200,41 @@ struct alignas(16) DevItem {
   uint32_t row_bytes;     // source bytes per row; 0 = contiguous (one row)
   uint32_t magic;         // division by row_bytes
   uint32_t shifts;        // s1 | s2 << 8
-  uint32_t flags;
+  uint32_t flags;         // bits 0-3 kind, 4-7 log2 of the vector bytes, kItemMerge
 };
 static_assert(sizeof(DevItem) == 64, "DevItem layout");
 
+constexpr uint32_t kItemMerge = 1u << 8;   // partly written lines are left to the L2 to merge
+
+// How a tile is moved.  The first five are the tiles of large tensors; "rows"
+// are strided.  ZERO rows are copied from a source of no bytes.
+enum : uint32_t {
+  kOpCopy = 0,         // contiguous, whole lines written through
+  kOpRows = 1,         // rows of a multiple of 16 bytes, whole lines written through
+  kOpRecast = 2,       // contiguous f32 -> f32 copy (where there is one) + bf16 copy
+  kOpZero = 3,
+  kOpRecastRows = 4,
+  kOpShifted = 5,      // contiguous copy into parts of lines, streamed
+  kOpRowsPart = 6,     // rows of a multiple of 16 bytes, streamed
+  kOpRows8 = 7,        // rows copied in 8-byte vectors, streamed
+  kOpRows4 = 8,
+  kOpNarrow = 9,       // vectors of less than 16 bytes otherwise
+  kOpWide = 10,        // 16-byte vectors otherwise
+  kOpFar = 11,         // rows 2 GiB or more apart
+};
+
+// The record of one tile.  A contiguous COPY or ZERO tile needs nothing else.
 struct alignas(8) DevTile {
-  uint64_t start;    // contiguous: byte offset in the item; strided: first row
+  uint64_t src;      // contiguous: address of its first source byte; strided: first row
+  uint64_t dst;      // contiguous: address of its first destination byte (0: none); strided: byte
+                     // column of the tile start in its first row
   uint32_t item;
-  uint32_t nbytes;   // source bytes in this tile
-  uint32_t c_base;   // strided: byte column of the tile start in its first row
-  uint32_t pad;
+  uint32_t info;     // bits 0-24 source bytes, 25-31 op
 };
 static_assert(sizeof(DevTile) == 24, "DevTile layout");
+
+constexpr uint32_t kTileOpBit = 25;
+constexpr uint32_t kTileBytesMask = (1u << kTileOpBit) - 1;
 
 // -------------------------------------------------------------- device code
 
@@ -228,123 +245,144 @@ template <> struct VecOf<4> { typedef unsigned int type; };
 template <> struct VecOf<2> { typedef unsigned short type; };
 template <> struct VecOf<1> { typedef unsigned char type; };
 
-// Global-memory accessors.  Descriptor tables carry addresses as integers,
-// so the global address space is stated here: the compiler then emits
-// global_load/global_store (VMEM only) instead of flat instructions, which
-// would also wait on the LDS counter.
+// A tile's source or destination bytes as a buffer resource: 32-bit offsets
+// from a base in scalar registers, and the hardware drops what lies outside
+// `bytes`, so lanes past a tile's end need no branch.
+typedef __amdgpu_buffer_rsrc_t Region;
+
+__device__ __forceinline__ Region region(uint64_t addr, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(addr), 0, bytes, 0x00027000);
+}
+
+// Bytes of the region a strided tile addresses, and an offset outside it for
+// the lanes past the tile's end.
+constexpr uint32_t kNearBytes = 1u << 31;
+constexpr uint32_t kNowhere = 0xfffffff0u;
+
+// Cache policies: the aux bits of gfx950's buffer instructions (2 = nt,
+// 16 = sc1).  Loads are non-temporal.  Stores of whole 64-byte lines write
+// through the L2: the lines then do not wait there for an eviction that
+// competes with the reads (flat copy of 2 GiB: 6.8 TB/s, nt 6.55; zero fill
+// 7.5, nt 6.5).  Lines that several waves or rows write in parts are left for
+// the L2 to merge, as streaming lines or, for short rows, as ordinary ones
+// (side by side rows of 4 bytes: through 3.0 TB/s, nt 3.6, ordinary 5.1; of
+// 36 kB + 16 bytes: 5.4, 5.9, 5.5).
+enum Policy : int {
+  kCached = 0,
+  kStream = 2,
+  kThrough = 16,
+};
+
+template <int VB, bool NT>
+__device__ __forceinline__ typename VecOf<VB>::type ld(Region r, uint32_t off) {
+  constexpr int aux = NT ? kStream : kCached;
+  typedef typename VecOf<VB>::type V;
+  if constexpr (VB == 16) return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, aux));
+  else if constexpr (VB == 8) return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, aux));
+  else if constexpr (VB == 4) return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, aux);
+  else if constexpr (VB == 2) return __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, aux);
+  else return __builtin_amdgcn_raw_buffer_load_b8(r, off, 0, aux);
+}
+
+template <int VB, Policy POLICY>
+__device__ __forceinline__ void st(Region r, uint32_t off, typename VecOf<VB>::type v) {
+  if constexpr (VB == 16) __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, POLICY);
+  else if constexpr (VB == 8) __builtin_amdgcn_raw_buffer_store_b64(v, r, off, 0, POLICY);
+  else if constexpr (VB == 4) __builtin_amdgcn_raw_buffer_store_b32(v, r, off, 0, POLICY);
+  else if constexpr (VB == 2) __builtin_amdgcn_raw_buffer_store_b16(v, r, off, 0, POLICY);
+  else __builtin_amdgcn_raw_buffer_store_b8(v, r, off, 0, POLICY);
+}
+
+// The same through 64-bit addresses (kOpFar).
 #define SR_GLOBAL __attribute__((address_space(1)))
 
-// Streaming (non-temporal) access applies to loads and stores separately
-// (compile-time knobs, both on by default).
-#ifndef SR_NT_LOADS
-#define SR_NT_LOADS 1
-#endif
-#ifndef SR_NT_STORES
-#define SR_NT_STORES 1
-#endif
-
-template <typename T, bool NT>
-__device__ __forceinline__ T ld(uint64_t addr) {
-  const SR_GLOBAL T* p = (const SR_GLOBAL T*)addr;
-  if constexpr (NT && SR_NT_LOADS) return __builtin_nontemporal_load(p);
-  else return *p;
+template <int VB>
+__device__ __forceinline__ typename VecOf<VB>::type ld_far(uint64_t addr) {
+  return __builtin_nontemporal_load((const SR_GLOBAL typename VecOf<VB>::type*)addr);
 }
 
-template <typename T, bool NT>
-__device__ __forceinline__ void st(uint64_t addr, T v) {
-  SR_GLOBAL T* p = (SR_GLOBAL T*)addr;
-  if constexpr (NT && SR_NT_STORES) __builtin_nontemporal_store(v, p);
-  else *p = v;
+template <int VB>
+__device__ __forceinline__ void st_far(uint64_t addr, typename VecOf<VB>::type v) {
+  __builtin_nontemporal_store(v, (SR_GLOBAL typename VecOf<VB>::type*)addr);
 }
 
-// Byte offsets, relative to the item's origins, of the source byte `b`
-// (counted from the start of the tile): source side, destination side and
-// bf16 side (half the destination column).  Contiguous items are one long
-// row; strided items divide by the row width.
-template <bool CONTIG>
-struct TileMap {
-  uint64_t start;
+// Row and column of the source byte `b` counted from the start of a strided
+// tile: a multiply-high division by the row width.
+struct RowMap {
   uint32_t c_base, width, magic, s1, s2;
-  uint64_t src_stride, dst_stride, dst2_stride;
 
-  __device__ __forceinline__ TileMap(const DevItem& it, const DevTile& t)
-      : start(t.start), c_base(t.c_base), width(it.row_bytes), magic(it.magic),
-        s1(it.shifts & 0xffu), s2(it.shifts >> 8), src_stride(it.src_stride),
-        dst_stride(it.dst_stride), dst2_stride(it.dst2_stride) {}
-
-  __device__ __forceinline__ void at(uint32_t b, uint64_t& so, uint64_t& dof) const {
-    if constexpr (CONTIG) {
-      so = start + b;
-      dof = so;
-    } else {
-      const uint32_t x = c_base + b;
-      const uint32_t q = div_apply(x, magic, s1, s2);
-      const uint64_t row = start + q;
-      const uint32_t col = x - q * width;
-      so = row * src_stride + col;
-      dof = row * dst_stride + col;
-    }
-  }
-
-  __device__ __forceinline__ void at(uint32_t b, uint64_t& so, uint64_t& dof, uint64_t& ho) const {
-    if constexpr (CONTIG) {
-      so = start + b;
-      dof = so;
-      ho = so >> 1;
-    } else {
-      const uint32_t x = c_base + b;
-      const uint32_t q = div_apply(x, magic, s1, s2);
-      const uint64_t row = start + q;
-      const uint32_t col = x - q * width;
-      so = row * src_stride + col;
-      dof = row * dst_stride + col;
-      ho = row * dst2_stride + (col >> 1);
-    }
+  __host__ __device__ __forceinline__ void at(uint32_t b, uint32_t& row, uint32_t& col) const {
+    const uint32_t x = c_base + b;
+    row = div_apply(x, magic, s1, s2);
+    col = x - row * width;
   }
 };
 
-// Copy one tile.  The main loop covers whole groups of kBlock * kUnroll
-// vectors with no bounds test, so each lane issues its kUnroll loads back to
-// back before the stores; the tail takes the remaining vectors one by one.
-template <int VB, bool NT, bool CONTIG>
-__device__ void copy_tile(const DevItem& it, const DevTile& t) {
-  typedef typename VecOf<VB>::type V;
-  constexpr int U = CONTIG ? kUnroll : kUnrollStrided;
-  const TileMap<CONTIG> map(it, t);
-  const uint32_t nvec = t.nbytes / VB;
-  constexpr uint32_t kStep = kBlock * U;
-  const uint32_t nfull = nvec / kStep * kStep;
-  for (uint32_t base = 0; base < nfull; base += kStep) {
-    V v[U];
-    uint64_t doff[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      uint64_t soff;
-      map.at((base + u * kBlock + threadIdx.x) * VB, soff, doff[u]);
-      v[u] = ld<V, NT>(it.src + soff);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) st<V, NT>(it.dst + doff[u], v[u]);
-  }
-  for (uint32_t i = nfull + threadIdx.x; i < nvec; i += kBlock) {
-    uint64_t soff, doff;
-    map.at(i * VB, soff, doff);
-    st<V, NT>(it.dst + doff, ld<V, NT>(it.src + soff));
-  }
+__device__ __forceinline__ RowMap row_map(const DevItem& it, uint32_t column) {
+  return {column, it.row_bytes, it.magic, it.shifts & 0xffu, it.shifts >> 8};
 }
 
-template <int VB, bool NT, bool CONTIG>
-__device__ void zero_tile(const DevItem& it, const DevTile& t) {
-  typedef typename VecOf<VB>::type V;
-  const TileMap<CONTIG> map(it, t);
-  const uint32_t nvec = t.nbytes / VB;
-  const V z = V(0);
-  for (uint32_t i = threadIdx.x; i < nvec; i += kBlock) {
-    uint64_t soff, doff;
-    map.at(i * VB, soff, doff);
-    st<V, NT>(it.dst + doff, z);
-  }
+// The 16-byte vector of a tile of rows of at least 16 bytes that starts at
+// tile byte `b`: its row and column, and whether its bytes go on in the next
+// row, where another vector starts at column 0.
+struct RowVec {
+  uint32_t row, col;
+  bool in, next;
+};
+
+__host__ __device__ __forceinline__ RowVec row_vec(const RowMap& rows, uint32_t b, uint32_t nbytes) {
+  RowVec v;
+  uint32_t col;
+  rows.at(b, v.row, col);
+  v.in = b < nbytes;
+  v.col = col < rows.width - 16u ? col : rows.width - 16u;
+  v.next = v.in && v.col != col && b + (rows.width - col) < nbytes;
+  return v;
 }
+
+// The offset of the 16-byte vector of a contiguous tile (16 bytes or more)
+// that starts at byte `b`; past the tile's end for lanes that have none.
+__host__ __device__ __forceinline__ uint32_t contiguous_vec(uint32_t b, uint32_t nbytes) {
+  return b < nbytes && b > nbytes - 16 ? nbytes - 16 : b;
+}
+
+// Where a vector of a tile goes: its offsets in the source, destination and
+// bf16 regions.  Lanes past the tile's end, and second vectors that are not
+// there, get an offset outside the regions.
+struct Place {
+  uint32_t src, dst, half;
+};
+
+// The places of the vectors `step` bytes apart in a tile: the first by a
+// division, the others by additions.  Width 0: one row.
+struct RowWalk {
+  uint32_t width, right, col;   // `step` on: some rows down, `right` columns on
+  Place at, by, wrap;           // wrap: to the next row's start
+
+  __host__ __device__ __forceinline__ RowWalk(const RowMap& rows, uint32_t b, uint32_t step, uint32_t ss, uint32_t ds,
+                                              uint32_t hs)
+      : width(0xffffffffu), right(step), col(b) {
+    uint32_t row = 0, down = 0;
+    if (rows.width) {
+      width = rows.width;
+      down = div_apply(step, rows.magic, rows.s1, rows.s2);
+      right = step - down * width;
+      rows.at(b, row, col);
+    }
+    at = {row * ss + col, row * ds + col, row * hs + (col >> 1)};
+    by = {down * ss + right, down * ds + right, down * hs + (right >> 1)};
+    wrap = {ss - width, ds - width, hs - (width >> 1)};
+  }
+
+  __host__ __device__ __forceinline__ void advance() {
+    col += right;
+    const bool over = col >= width;
+    col -= over ? width : 0;
+    at.src += by.src + (over ? wrap.src : 0);
+    at.dst += by.dst + (over ? wrap.dst : 0);
+    at.half += by.half + (over ? wrap.half : 0);
+  }
+};
 
 // float -> bfloat16, round to nearest, ties to even; NaN -> 0x7FC0.
 // This is the standard integer rounding of the upper half-word: add
@@ -366,100 +404,294 @@ __device__ __forceinline__ typename VecOf<2 * NE>::type to_bf16(typename VecOf<4
   return h;
 }
 
-// f32 region -> f32 copy (when the item has one) + bf16 RNE copy.
-template <int NE, bool NT, bool CONTIG>
-__device__ void recast_tile(const DevItem& it, const DevTile& t) {
-  constexpr int SB = 4 * NE;                 // source (f32) bytes per lane vector
-  typedef typename VecOf<SB>::type VS;       // NE f32
-  typedef typename VecOf<2 * NE>::type VH;   // NE bf16
-  const TileMap<CONTIG> map(it, t);
-  const uint32_t nvec = t.nbytes / SB;
-  const bool has_dst = (it.flags >> 8) & 1u;
-  constexpr int U = kUnrollStrided;
-  constexpr uint32_t kStep = kBlock * U;
-  const uint32_t nfull = nvec / kStep * kStep;
-  for (uint32_t base = 0; base < nfull; base += kStep) {
-    VS v[U];
-    uint64_t doff[U], hoff[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      uint64_t soff;
-      map.at((base + u * kBlock + threadIdx.x) * SB, soff, doff[u], hoff[u]);
-      v[u] = ld<VS, NT>(it.src + soff);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (has_dst) st<VS, NT>(it.dst + doff[u], v[u]);
-      st<VH, NT>(it.dst2 + hoff[u], to_bf16<NE>(v[u]));
+// What a tile reads and writes; a region of no bytes takes no store.
+struct Regions {
+  Region src, dst, half;
+};
+
+// Stores a loaded vector: COPY the bytes, RECAST also the rounded ones.
+template <uint32_t KIND, int VB, Policy POLICY>
+__device__ __forceinline__ void put(const Regions& r, const Place& at, typename VecOf<VB>::type v) {
+  st<VB, POLICY>(r.dst, at.dst, v);
+  if constexpr (KIND == kKindRecast) st<VB / 2, POLICY>(r.half, at.half, to_bf16<VB / 4>(v));
+}
+
+// The tile records this far ahead of a workgroup's own are read into the
+// die's L2 (one read per kAheadStep records, which span less than a cache
+// line), so that a record is there when its workgroup starts.  The read is
+// issued behind the tile's loads and done with before its stores: a wait
+// after them would hold the wave until they are written.  256 records cover a
+// die's tiles in flight twice over (flat copy of 2 GiB: 6.40 TB/s without,
+// 6.69 with 256 or 512 ahead, 6.47 with 2048).
+constexpr uint32_t kAhead = 256;
+constexpr uint32_t kAheadStep = 4;
+
+struct Ahead {
+  const DevTile* tiles;
+  uint32_t i, n, lane;
+  __device__ __forceinline__ void touch() const {
+    if (lane >= kBlock - 64 && i % kAheadStep == 0 && i + kAhead < n) {
+      const uint32_t x = __hip_atomic_load(&tiles[i + kAhead].info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      asm volatile("" ::"v"(x));
     }
   }
-  for (uint32_t i = nfull + threadIdx.x; i < nvec; i += kBlock) {
-    uint64_t soff, doff, hoff;
-    map.at(i * SB, soff, doff, hoff);
-    const VS v = ld<VS, NT>(it.src + soff);
-    if (has_dst) st<VS, NT>(it.dst + doff, v);
-    st<VH, NT>(it.dst2 + hoff, to_bf16<NE>(v));
+};
+
+// A tile of at least 16 contiguous bytes, at any alignment: 16 bytes per
+// lane, the last vector moved back to end with the tile (it then writes
+// bytes of its neighbour again, with the same values).
+template <uint32_t KIND, bool NT, Policy POLICY>
+__device__ __forceinline__ void contiguous_tile(const Regions& r, uint32_t nbytes, const Ahead& ahead) {
+  for (uint32_t base = 0; base < nbytes; base += kPassBytes) {
+    const uint32_t off = contiguous_vec(base + ahead.lane * 16, nbytes);
+    VecOf<16>::type v(0);
+    if constexpr (KIND != kKindZero) {
+      v = ld<16, NT>(r.src, off);
+      if (base == 0) ahead.touch();
+    }
+    put<KIND, 16, POLICY>(r, Place{off, off, off >> 1}, v);
   }
 }
 
-template <bool NT, bool CONTIG>
-__device__ __forceinline__ void exec_tile(const DevItem& it, const DevTile& t) {
-  const uint32_t kind = it.flags & 0xfu;
-  const uint32_t lv = (it.flags >> 4) & 0xfu;
-  if (kind == kKindCopy) {
-    switch (lv) {
-      case 4: copy_tile<16, NT, CONTIG>(it, t); break;
-      case 3: copy_tile<8, NT, CONTIG>(it, t); break;
-      case 2: copy_tile<4, NT, CONTIG>(it, t); break;
-      case 1: copy_tile<2, NT, CONTIG>(it, t); break;
-      default: copy_tile<1, NT, CONTIG>(it, t); break;
+// A tile of rows of a multiple of 16 bytes, at any alignment: 16 bytes per lane.
+template <uint32_t KIND, bool NT, Policy POLICY>
+__device__ __forceinline__ void rows_tile(const Regions& r, const DevItem& it, uint32_t column, uint32_t nbytes,
+                                          const Ahead& ahead) {
+  const RowMap rows = row_map(it, column);
+  const uint32_t ss = uint32_t(it.src_stride), ds = uint32_t(it.dst_stride), hs = uint32_t(it.dst2_stride);
+  for (uint32_t base = 0; base < nbytes; base += kPassBytes) {
+    const uint32_t b = base + ahead.lane * 16;
+    uint32_t row, col;
+    rows.at(b, row, col);
+    const bool in = b < nbytes;
+    const Place at = {in ? row * ss + col : kNowhere, in ? row * ds + col : kNowhere,
+                      in ? row * hs + (col >> 1) : kNowhere};
+    const VecOf<16>::type v = ld<16, NT>(r.src, at.src);
+    if (base == 0) ahead.touch();
+    put<KIND, 16, POLICY>(r, at, v);
+  }
+}
+
+// The forms below branch at run time where that saves code: with a variant
+// of every form for every kind and policy the kernel grew from 20 to 46 KB,
+// and the paths above lost 3% to its instruction fetches.
+#define SR_BY_POLICY(MERGE, CALL)       \
+  do {                                  \
+    if (NT && !(MERGE)) CALL(kStream);  \
+    else CALL(kCached);                 \
+  } while (0)
+
+// The regions of a strided tile (or of a contiguous piece that is one tile,
+// from its origin).
+__device__ __forceinline__ Regions row_regions(const DevItem& it, uint64_t row) {
+  return {region(it.src + row * it.src_stride, it.src ? kNearBytes : 0),
+          region(it.dst + row * it.dst_stride, it.dst ? kNearBytes : 0),
+          region(it.dst2 + row * it.dst2_stride, it.dst2 ? kNearBytes : 0)};
+}
+
+// 16-byte vectors at any alignment, rows of at least 16 bytes.  A vector
+// that runs over the end of its row (rows that are no multiple of 16 bytes;
+// not RECAST) becomes two, the last 16 bytes of that row and the first 16 of
+// the next; the bytes that neighbouring lanes write too have the same values.
+template <bool NT>
+__device__ __forceinline__ void wide_tile(const DevItem& it, const DevTile& t, uint32_t nbytes, const Ahead& ahead) {
+  const bool strided = it.row_bytes != 0, recast = (it.flags & 0xfu) == kKindRecast;
+  const Regions r = strided ? row_regions(it, t.src)
+                            : Regions{region(t.src, it.src ? nbytes : 0), region(t.dst, t.dst ? nbytes : 0),
+                                      region(it.dst2 + ((t.src - it.src) >> 1), it.dst2 ? nbytes >> 1 : 0)};
+  const RowMap rows = row_map(it, uint32_t(t.dst));
+  const uint32_t ss = uint32_t(it.src_stride), ds = uint32_t(it.dst_stride), hs = uint32_t(it.dst2_stride);
+  for (uint32_t base = 0; base < nbytes; base += kPassBytes) {
+    const uint32_t b = base + ahead.lane * 16;
+    Place at, at2{kNowhere, kNowhere, kNowhere};
+    if (strided) {
+      const RowVec x = row_vec(rows, b, nbytes);
+      if (x.in) at = {x.row * ss + x.col, x.row * ds + x.col, x.row * hs + (x.col >> 1)};
+      else at = at2;
+      if (x.next) at2 = {(x.row + 1) * ss, (x.row + 1) * ds, kNowhere};
+    } else {
+      const uint32_t off = contiguous_vec(b, nbytes);
+      at = {off, off, off >> 1};
     }
-  } else if (kind == kKindRecast) {
-    if (lv == 2) recast_tile<4, NT, CONTIG>(it, t);
-    else recast_tile<1, NT, CONTIG>(it, t);
+    const VecOf<16>::type v = ld<16, NT>(r.src, at.src), w = ld<16, NT>(r.src, at2.src);
+    const VecOf<8>::type h = to_bf16<4>(v);
+    if (base == 0) ahead.touch();
+#define SR_PUT(POLICY)                                \
+  do {                                                \
+    st<16, POLICY>(r.dst, at.dst, v);                 \
+    if (recast) st<8, POLICY>(r.half, at.half, h);    \
+    else st<16, POLICY>(r.dst, at2.dst, w);           \
+  } while (0)
+    SR_BY_POLICY(it.flags & kItemMerge, SR_PUT);
+#undef SR_PUT
+  }
+}
+
+// Vectors of the widest aligned type that divides the rows (RECAST: one
+// element).  A wave takes consecutive bytes, U vectors per lane a wave's
+// width apart: each vector's lines are then written by one wave (side by
+// side f32 rows of 16396 bytes: 5.7 TB/s, with the vectors of a lane a
+// workgroup's width apart 5.2).
+template <uint32_t KIND, int VB, bool NT, Policy POLICY>
+__device__ __forceinline__ void narrow_vectors(const Regions& r, const DevItem& it, uint32_t column, uint32_t nbytes,
+                                               const Ahead& ahead) {
+  constexpr int U = VB == 8 ? 2 : 4;
+  constexpr uint32_t kStep = 64 * VB;
+  const RowMap rows = row_map(it, column);
+  for (uint32_t base = 0; base < nbytes; base += kBlock * VB * U) {
+    uint32_t b = base + (ahead.lane >> 6) * (U * kStep) + (ahead.lane & 63) * VB;
+    RowWalk walk(rows, b, kStep, uint32_t(it.src_stride), uint32_t(it.dst_stride), uint32_t(it.dst2_stride));
+    Place at[U];
+    typename VecOf<VB>::type v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool in = b < nbytes;
+      at[u] = {kNowhere, in ? walk.at.dst : kNowhere, in ? walk.at.half : kNowhere};
+      v[u] = ld<VB, NT>(r.src, in ? walk.at.src : kNowhere);
+      b += kStep;
+      walk.advance();
+    }
+    if (base == 0) ahead.touch();
+#pragma unroll
+    for (int u = 0; u < U; ++u) put<KIND, VB, POLICY>(r, at[u], v[u]);
+  }
+}
+
+template <bool NT>
+__device__ __forceinline__ void narrow_tile(const DevItem& it, const DevTile& t, uint32_t nbytes, const Ahead& ahead) {
+  const bool strided = it.row_bytes != 0, merge = !NT || (it.flags & kItemMerge);
+  const uint32_t lv = (it.flags >> 4) & 0xfu, column = strided ? uint32_t(t.dst) : 0;
+  const Regions r = row_regions(it, strided ? t.src : 0);
+  constexpr Policy kPart = NT ? kStream : kCached;
+  if ((it.flags & 0xfu) == kKindRecast) {
+    if (merge) narrow_vectors<kKindRecast, 4, NT, kCached>(r, it, column, nbytes, ahead);
+    else narrow_vectors<kKindRecast, 4, NT, kPart>(r, it, column, nbytes, ahead);
+  } else if (lv == 3) {   // streamed: kOpRows8, kOpRows4, or one small piece
+    narrow_vectors<kKindCopy, 8, NT, kCached>(r, it, column, nbytes, ahead);
+  } else if (lv == 2) {
+    narrow_vectors<kKindCopy, 4, NT, kCached>(r, it, column, nbytes, ahead);
+  } else if (lv == 1) {
+    if (merge) narrow_vectors<kKindCopy, 2, NT, kCached>(r, it, column, nbytes, ahead);
+    else narrow_vectors<kKindCopy, 2, NT, kPart>(r, it, column, nbytes, ahead);
   } else {
-    switch (lv) {
-      case 4: zero_tile<16, NT, CONTIG>(it, t); break;
-      case 3: zero_tile<8, NT, CONTIG>(it, t); break;
-      case 2: zero_tile<4, NT, CONTIG>(it, t); break;
-      case 1: zero_tile<2, NT, CONTIG>(it, t); break;
-      default: zero_tile<1, NT, CONTIG>(it, t); break;
+    if (merge) narrow_vectors<kKindCopy, 1, NT, kCached>(r, it, column, nbytes, ahead);
+    else narrow_vectors<kKindCopy, 1, NT, kPart>(r, it, column, nbytes, ahead);
+  }
+}
+
+// One vector at a time through 64-bit addresses: strided items whose tiles
+// span 2 GiB or more of an object (a few bytes of very long rows).
+__device__ __forceinline__ void far_tile(const DevItem& it, const DevTile& t, uint32_t nbytes, uint32_t lane) {
+  const uint32_t lv = (it.flags >> 4) & 0xfu, kind = it.flags & 0xfu;
+  const RowMap rows = row_map(it, uint32_t(t.dst));
+  for (uint32_t b = lane << lv; b < nbytes; b += kBlock << lv) {
+    uint32_t row, col;
+    rows.at(b, row, col);
+    const uint64_t q = t.src + row;
+    const uint64_t from = it.src + q * it.src_stride + col, to = it.dst + q * it.dst_stride + col;
+    const uint64_t half = it.dst2 + q * it.dst2_stride + (col >> 1);
+    if (kind == kKindRecast) {
+      if (lv == 4) {
+        const VecOf<16>::type v = ld_far<16>(from);
+        if (it.dst) st_far<16>(to, v);
+        st_far<8>(half, to_bf16<4>(v));
+      } else {
+        const uint32_t v = ld_far<4>(from);
+        if (it.dst) st_far<4>(to, v);
+        st_far<2>(half, to_bf16<1>(v));
+      }
+    } else if (lv == 4) {
+      st_far<16>(to, kind == kKindZero ? VecOf<16>::type(0) : ld_far<16>(from));
+    } else if (lv == 3) {
+      st_far<8>(to, kind == kKindZero ? VecOf<8>::type(0) : ld_far<8>(from));
+    } else if (lv == 2) {
+      st_far<4>(to, kind == kKindZero ? 0u : ld_far<4>(from));
+    } else if (lv == 1) {
+      st_far<2>(to, kind == kKindZero ? (unsigned short)0 : ld_far<2>(from));
+    } else {
+      st_far<1>(to, kind == kKindZero ? (unsigned char)0 : ld_far<1>(from));
     }
   }
 }
 
+// The tile at each position of the grid.  With `seg` non-zero the list is
+// cut into kXcds segments of `seg` tiles and position p takes tile p / kXcds
+// of segment p % kXcds: each die walks one contiguous part of the list, and
+// of the records.  Positions p, p + stride, ... below n_pos are this
+// workgroup's; `stride` is the grid.
 template <bool NT>
-__device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items,
-                                           const DevTile* __restrict__ tiles, uint32_t n_tiles) {
-  for (uint32_t ti = blockIdx.x; ti < n_tiles; ti += gridDim.x) {
-    const DevTile t = tiles[ti];
-    const DevItem it = items[t.item];
-    if (it.row_bytes == 0) exec_tile<NT, true>(it, t);
-    else exec_tile<NT, false>(it, t);
+__device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, const DevTile* __restrict__ tiles,
+                                           uint32_t n_tiles, uint32_t seg, uint32_t n_pos, uint32_t stride) {
+  uint32_t p = blockIdx.x;
+  do {
+    const uint32_t i = seg ? (p % kXcds) * seg + p / kXcds : p;
+    if (i < n_tiles) {
+      const DevTile t = tiles[i];
+      // made anew for each tile: what a path derives from it would otherwise
+      // be computed for all paths before the loop, and held
+      uint32_t lane = threadIdx.x;
+      asm volatile("" : "+v"(lane));
+      const Ahead ahead{tiles, i, n_tiles, lane};
+      const uint32_t op = t.info >> kTileOpBit, nbytes = t.info & kTileBytesMask;
+      constexpr Policy kWhole = NT ? kThrough : kCached, kPartial = NT ? kStream : kCached;
+      const Region none = region(0, 0);
+      if (__builtin_expect(op == kOpCopy, 1)) {
+        contiguous_tile<kKindCopy, NT, kWhole>(Regions{region(t.src, nbytes), region(t.dst, nbytes), none}, nbytes,
+                                               ahead);
+      } else if (__builtin_expect(op == kOpRows, 1)) {
+        const DevItem it = items[t.item];
+        rows_tile<kKindCopy, NT, kWhole>(Regions{region(it.src + t.src * it.src_stride, it.src ? kNearBytes : 0),
+                                                 region(it.dst + t.src * it.dst_stride, kNearBytes), none},
+                                         it, uint32_t(t.dst), nbytes, ahead);
+      } else if (__builtin_expect(op == kOpRecast, 1)) {
+        const uint64_t half = items[t.item].dst2 + ((t.src - items[t.item].src) >> 1);
+        contiguous_tile<kKindRecast, NT, kWhole>(
+            Regions{region(t.src, nbytes), region(t.dst, t.dst ? nbytes : 0), region(half, nbytes >> 1)}, nbytes,
+            ahead);
+      } else if (__builtin_expect(op == kOpZero, 1)) {
+        contiguous_tile<kKindZero, NT, kWhole>(Regions{none, region(t.dst, nbytes), none}, nbytes, ahead);
+      } else if (__builtin_expect(op == kOpRecastRows, 1)) {
+        const DevItem it = items[t.item];
+        rows_tile<kKindRecast, NT, kWhole>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
+      } else if (op == kOpShifted) {
+        contiguous_tile<kKindCopy, NT, kPartial>(Regions{region(t.src, nbytes), region(t.dst, nbytes), none}, nbytes,
+                                                 ahead);
+      } else if (op == kOpRowsPart) {
+        const DevItem it = items[t.item];
+        rows_tile<kKindCopy, NT, kPartial>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
+      } else if (op == kOpRows8) {
+        const DevItem it = items[t.item];
+        narrow_vectors<kKindCopy, 8, NT, kPartial>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
+      } else if (op == kOpRows4) {
+        const DevItem it = items[t.item];
+        narrow_vectors<kKindCopy, 4, NT, kPartial>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
+      } else if (op == kOpNarrow) {
+        narrow_tile<NT>(items[t.item], t, nbytes, ahead);
+      } else if (op == kOpWide) {
+        wide_tile<NT>(items[t.item], t, nbytes, ahead);
+      } else {
+        far_tile(items[t.item], t, nbytes, lane);
+      }
+    }
+    p += stride;
+  } while (p < n_pos);
+}
+
+// Three entry points with one body, so profiles tell the phases apart.  Eight
+// waves per SIMD (two workgroups per compute unit) need at most 64 vector
+// registers and, the trap handler's 16 included, 96 scalar ones each: with
+// 84 of its own the kernel ran one workgroup per unit and lost 15%.
+#define SR_COPY_KERNEL(NAME)                                                                                      \
+  template <bool NT>                                                                                              \
+  __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(8))) void NAME(    \
+      const DevItem* __restrict__ items, const DevTile* __restrict__ tiles, uint32_t n_tiles, uint32_t seg,       \
+      uint32_t n_pos, uint32_t stride) {                                                                          \
+    exec_tiles<NT>(items, tiles, n_tiles, seg, n_pos, stride);                                                    \
   }
-}
-
-// Two entry points with one body, so profiles tell the phases apart.
-template <bool NT>
-__global__ __launch_bounds__(kBlock) void sr_pack_kernel(const DevItem* __restrict__ items,
-                                                         const DevTile* __restrict__ tiles,
-                                                         uint32_t n_tiles) {
-  exec_tiles<NT>(items, tiles, n_tiles);
-}
-
-template <bool NT>
-__global__ __launch_bounds__(kBlock) void sr_unpack_kernel(const DevItem* __restrict__ items,
-                                                           const DevTile* __restrict__ tiles,
-                                                           uint32_t n_tiles) {
-  exec_tiles<NT>(items, tiles, n_tiles);
-}
-
-template <bool NT>
-__global__ __launch_bounds__(kBlock) void sr_gather_kernel(const DevItem* __restrict__ items,
-                                                           const DevTile* __restrict__ tiles,
-                                                           uint32_t n_tiles) {
-  exec_tiles<NT>(items, tiles, n_tiles);
-}
+SR_COPY_KERNEL(sr_pack_kernel)
+SR_COPY_KERNEL(sr_unpack_kernel)
+SR_COPY_KERNEL(sr_gather_kernel)
+#undef SR_COPY_KERNEL
 
 // ------------------------------------------------- device-side plan binding
 // The host keeps O(pieces) descriptors and the prefix sum of their tile
@@ -467,24 +699,16 @@ __global__ __launch_bounds__(kBlock) void sr_gather_kernel(const DevItem* __rest
 // absolute-address item table are computed on the GPU from them:
 //   sr_offsets_kernel   per peer: exclusive prefix sum of the 256-byte
 //                       rounded payloads of its pieces, in piece order;
-//   sr_tile_emit_kernel one workgroup per item writes its tiles, placed in
-//                       the XCD-interleaved order, and on a phase's first
-//                       launch binds the item as sr_bind_kernel does;
-//   sr_bind_kernel      one lane per item: caller pointers + offsets ->
-//                       DevItem (addresses, vector width); later launches
-//                       with other pointers.
+//   sr_tile_emit_kernel one workgroup per chunk of an item's tiles writes
+//                       their records, bound to the caller's pointers; again
+//                       for other pointers.
 
 // Pointer-independent item descriptor (device resident, uploaded once).
 enum : uint32_t {
   kRelSrcBuf = 1u << 16,   // source side is a peer buffer at the piece's offset
   kRelDstBuf = 1u << 17,   // destination side is a peer buffer at the piece's offset
-  kRelTileShiftBit = 20,   // bits 20-23: the item's tiles are tile_bytes >> this
+  kRelFar = 1u << 18,      // kOpFar
 };
-
-// log2 of an item's tile size in source bytes.
-__host__ __device__ inline uint32_t item_tile_shift(uint32_t kind, uint32_t tile_shift) {
-  return tile_shift - ((kind >> kRelTileShiftBit) & 0xfu);
-}
 
 struct alignas(8) DevRel {
   uint64_t src_off;        // byte offset of the region origin in its object
@@ -497,8 +721,7 @@ struct alignas(8) DevRel {
   uint32_t row_bytes;      // 0 = contiguous
   uint32_t magic;
   uint32_t shifts;
-  uint32_t kind;           // bits 0-7 kind, 8-15 element bytes, kRelSrcBuf / kRelDstBuf,
-                           // bits 20-23 tile size reduction (kRelTileShiftBit)
+  uint32_t kind;           // bits 0-7 kind, 8-15 element bytes, kRelSrcBuf / kRelDstBuf / kRelFar
   int32_t src_slot;        // index into the phase's pointer table, -1 = none
   int32_t dst_slot;
   int32_t dst2_slot;
@@ -590,15 +813,35 @@ __host__ __device__ inline uint32_t log2u(uint32_t v) {
   return l;
 }
 
+// The narrowest rows that move as 16-byte vectors at any alignment rather
+// than as aligned vectors of `vb` bytes, by whether the destination is dense.
+// Measured on 1 GiB halves of bf16 (vb 2) and u8 (vb 1) rows, TB/s, narrow
+// against 16-byte: side by side rows of 66 bytes 3.2 / 3.7-4.0, 514 bytes
+// 3.2 / 4.8; dense rows of 202 bytes 4.0 / 3.6, 514 bytes 4.2 / 4.9; u8 side
+// by side of 17 bytes 2.0 / 3.1, dense of 33 bytes 2.5 / 2.4, 101 bytes
+// 2.5 / 2.7.  Rows that are 4-byte aligned stay narrow at every width (f32
+// rows of 2732 bytes, dense: 5.6 / 5.2).
+__host__ __device__ inline uint32_t ragged_from(uint32_t vb, bool dense) {
+  if (vb == 1) return dense ? 64 : 16;
+  if (vb == 2) return dense ? 400 : 64;
+  return 0xffffffffu;
+}
+
+// Rows of a destination that is not dense leave their lines to be merged
+// when they are shorter than this, RECAST at any width: f32 rows of 260 bytes
+// streamed 4.4, merged 4.9 TB/s; of 800 bytes 5.7 / 5.5; ZERO rows of 192
+// bytes 2.9 / 3.5, of 400 bytes 4.7 / 3.5; RECAST of 800 bytes 5.3 / 5.6.
+constexpr uint32_t kMergeBelow = 512, kMergeZeroBelow = 384;
+
 // The item of descriptor `h`: its object addresses resolved from `ptrs`,
 // the phase's pointer table (source objects, then destination objects),
-// and `offset`, the per-piece buffer offsets from sr_offsets_kernel, and
-// the widest vector access its addresses and sizes allow.
+// and `offset`, the per-piece buffer offsets from sr_offsets_kernel; the
+// vector and the op of its tiles.
 __device__ __forceinline__ DevItem bind_item(const DevRel& h, const uint64_t* __restrict__ ptrs,
-                                             const uint64_t* __restrict__ offset) {
+                                             const uint64_t* __restrict__ offset, uint32_t& op) {
   const uint32_t kind = h.kind & 0xffu;
-  const uint32_t esize = (h.kind >> 8) & 0xffu;
   const bool contiguous = h.row_bytes == 0;
+  const bool far = (h.kind & kRelFar) != 0;
   DevItem d;
   d.src = h.src_slot >= 0 ? ptrs[h.src_slot] + ((h.kind & kRelSrcBuf) ? offset[h.piece] : h.src_off) : 0;
   d.dst = h.dst_slot >= 0 ? ptrs[h.dst_slot] + ((h.kind & kRelDstBuf) ? offset[h.piece] : h.dst_off) : 0;
@@ -609,66 +852,59 @@ __device__ __forceinline__ DevItem bind_item(const DevRel& h, const uint64_t* __
   d.row_bytes = h.row_bytes;
   d.magic = h.magic;
   d.shifts = h.shifts;
-  uint32_t lv = 0;
-  if (kind == kKindCopy) {
-    uint64_t acc = d.src | d.dst;
-    acc |= contiguous ? h.total : (uint64_t(h.row_bytes) | h.src_stride | h.dst_stride);
-    lv = log2u(pick_vb(acc, esize));
-  } else if (kind == kKindZero) {
-    uint64_t acc = d.dst;
-    acc |= contiguous ? h.total : (uint64_t(h.row_bytes) | h.dst_stride);
-    lv = log2u(pick_vb(acc, esize));
-  } else {
-    // RECAST: 4 f32 per lane when the f32 sides are 16-byte and the bf16
-    // side 8-byte aligned, otherwise one element per lane.
-    const bool has_dst = h.dst_slot >= 0;
-    bool wide = ((d.src | (has_dst ? d.dst : 0)) & 15) == 0 && (d.dst2 & 7) == 0;
-    if (contiguous) {
-      wide = wide && (h.total & 15) == 0;
-    } else {
-      wide = wide && (h.row_bytes & 15) == 0 && (h.src_stride & 15) == 0 &&
-             (!has_dst || (h.dst_stride & 15) == 0) && (h.dst2_stride & 7) == 0;
-    }
-    lv = wide ? 2 : 0;
-  }
-  d.flags = kind | (lv << 4) | ((kind == kKindRecast && h.dst_slot >= 0) ? (1u << 8) : 0u);
-  return d;
-}
+  const uint64_t width = contiguous ? h.total : h.row_bytes;
+  // the destination's rows lie end to end
+  const bool dense = contiguous || ((h.dst_slot < 0 || h.dst_stride == h.row_bytes) &&
+                                    (h.dst2_slot < 0 || h.dst2_stride * 2 == h.row_bytes));
 
-// Tile i of the item-ordered list goes to position pos(i).  With `ways`
-// segments of seg = ceil(n/ways) tiles (q full segments and a last one of
-// r tiles), tile j of segment s is dispatched at j*q + min(j, r) + s: the
-// list is read column by column, so consecutive workgroups -- which the
-// hardware deals to the 8 XCDs in turn -- take one tile from each segment.
-__device__ __forceinline__ uint64_t xcd_position(uint64_t i, uint64_t seg, uint64_t q, uint64_t r) {
-  const uint64_t s = i / seg;
-  const uint64_t j = i - s * seg;
-  return j * q + (j < r ? j : r) + s;
+  // the widest vector that all addresses and sizes are aligned for (RECAST:
+  // four elements, or one), or 16 bytes at any alignment
+  uint64_t at = d.src | d.dst | width;
+  if (!contiguous) at |= h.src_stride | h.dst_stride;
+  uint32_t lv = log2u(pick_vb(at, kind == kKindRecast ? 4 : (h.kind >> 8) & 0xffu));
+  if (kind == kKindRecast) {
+    const uint64_t half = d.dst2 | (contiguous ? 0 : h.dst2_stride);
+    if (lv < 4 || (half & 7)) lv = contiguous && width >= 16 ? 4 : 2;
+  } else if (!far && width >= (contiguous || kind == kKindZero ? 16 : ragged_from(1u << lv, dense))) {
+    lv = 4;
+  }
+
+  // 16-byte vectors into whole lines: of each row, or of a dense destination
+  uint64_t line = d.dst | d.dst2;
+  if (!dense) {
+    line |= h.row_bytes | h.dst_stride | h.dst2_stride;
+    if (kind == kKindRecast) line |= h.row_bytes >> 1;
+  }
+  const bool merge =
+      !dense && (kind == kKindRecast || h.row_bytes < (kind == kKindZero ? kMergeZeroBelow : kMergeBelow));
+  const bool whole = (line & 63) == 0;
+  if (far) op = kOpFar;
+  else if (lv < 4 && (contiguous || merge || kind == kKindRecast || lv < 2)) op = kOpNarrow;
+  else if (lv < 4) op = lv == 3 ? kOpRows8 : kOpRows4;
+  else if (contiguous && whole) op = kind == kKindCopy ? kOpCopy : kind == kKindZero ? kOpZero : kOpRecast;
+  else if (contiguous && kind == kKindCopy) op = kOpShifted;
+  else if (!contiguous && whole && h.row_bytes % 16 == 0) op = kind == kKindRecast ? kOpRecastRows : kOpRows;
+  else if (!contiguous && !merge && kind != kKindRecast && h.row_bytes % 16 == 0) op = kOpRowsPart;
+  else op = kOpWide;
+  d.flags = kind | (lv << 4) | (merge ? kItemMerge : 0u);
+  return d;
 }
 
 // One workgroup per emit chunk -- up to kEmitTiles consecutive tiles of one
 // item (chunks[c] = {item, chunk index}; every item has at least one) --
-// writes those tiles (tile_base[k] = tiles of items 0..k-1, computed with the
-// descriptors on the host).  With `items` non-null, lane 0 of an item's
-// first chunk also binds the item to the pointer table `ptrs` (and the
-// buffer offsets `offset`), as sr_bind_kernel does: a phase's first launch
-// builds both tables in one kernel.
+// writes those tiles' records, in list order (tile_base[k] = tiles of items
+// 0..k-1, computed with the descriptors on the host), bound to the pointer
+// table `ptrs` (and the buffer offsets `offset`).  Lane 0 of an item's first
+// chunk also writes the bound item.
 __global__ __launch_bounds__(kSetupBlock) void sr_tile_emit_kernel(
     const DevRel* __restrict__ rel, const uint64_t* __restrict__ tile_base, const EmitChunk* __restrict__ chunks,
-    uint32_t n_chunks, uint32_t tile_shift, uint64_t n_tiles, uint32_t ways, DevTile* __restrict__ tiles,
-    const uint64_t* __restrict__ ptrs, const uint64_t* __restrict__ offset, DevItem* __restrict__ items) {
-  uint64_t seg = 1, q = n_tiles, r = 0;
-  if (ways > 1) {
-    seg = (n_tiles + ways - 1) / ways;
-    q = n_tiles / seg;
-    r = n_tiles - q * seg;
-  }
+    uint32_t n_chunks, uint32_t tile_shift, DevTile* __restrict__ tiles, const uint64_t* __restrict__ ptrs,
+    const uint64_t* __restrict__ offset, DevItem* __restrict__ items) {
   for (uint32_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
     const uint32_t k = chunks[c].item;
     const uint64_t j0 = uint64_t(chunks[c].chunk) * kEmitTiles;
     const uint64_t total = rel[k].total;
     const uint32_t width = rel[k].row_bytes;
-    const uint32_t sh = item_tile_shift(rel[k].kind, tile_shift);
     const uint64_t cnt = tile_base[k + 1] - tile_base[k];
     // Items of a group have equal tile counts; tile j of member m goes to
     // group_start + j*M + m, so the members' tiles over the same rows are
@@ -676,37 +912,32 @@ __global__ __launch_bounds__(kSetupBlock) void sr_tile_emit_kernel(
     const uint64_t gm = rel[k].group_index;
     const uint64_t gsize = rel[k].group_size;
     const uint64_t b = tile_base[k] - gm * cnt + gm;
-    if (items != nullptr && j0 == 0 && threadIdx.x == 0) items[k] = bind_item(rel[k], ptrs, offset);
+    uint32_t op;
+    const DevItem item = bind_item(rel[k], ptrs, offset, op);
+    if (j0 == 0 && threadIdx.x == 0) items[k] = item;
+    const uint32_t info = op << kTileOpBit;
     const uint64_t j1 = cnt < j0 + kEmitTiles ? cnt : j0 + kEmitTiles;
     for (uint64_t j = j0 + threadIdx.x; j < j1; j += kSetupBlock) {
-      const uint64_t start = j << sh;
-      const uint64_t left = total - start;
+      uint64_t start = j << tile_shift;
+      uint64_t n = total - start < (uint64_t(1) << tile_shift) ? total - start : (uint64_t(1) << tile_shift);
+      if (width == 0 && total >= 16 && n < 16) {   // a whole vector, from the tile before
+        start -= 16 - n;
+        n = 16;
+      }
       DevTile t;
       t.item = k;
-      t.nbytes = uint32_t(left < (uint64_t(1) << sh) ? left : (uint64_t(1) << sh));
-      t.pad = 0;
+      t.info = info | uint32_t(n);
       if (width == 0) {
-        t.start = start;
-        t.c_base = 0;
+        t.src = item.src + start;
+        t.dst = item.dst ? item.dst + start : 0;
       } else {
         const uint64_t row = start / width;
-        t.start = row;
-        t.c_base = uint32_t(start - row * width);
+        t.src = row;
+        t.dst = start - row * width;
       }
-      const uint64_t i = b + j * gsize;
-      tiles[ways > 1 ? xcd_position(i, seg, q, r) : i] = t;
+      tiles[b + j * gsize] = t;
     }
   }
-}
-
-__global__ __launch_bounds__(kSetupBlock) void sr_bind_kernel(const DevRel* __restrict__ rel,
-                                                              uint32_t n,
-                                                              const uint64_t* __restrict__ ptrs,
-                                                              const uint64_t* __restrict__ offset,
-                                                              DevItem* __restrict__ items) {
-  const uint32_t k = blockIdx.x * kSetupBlock + threadIdx.x;
-  if (k >= n) return;
-  items[k] = bind_item(rel[k], ptrs, offset);
 }
 
 // ----------------------------------------------------------- host structures
@@ -733,9 +964,10 @@ struct HostItem {
 struct Phase {
   std::vector<HostItem> items;          // in piece order while the plan is built
   std::vector<DevRel> rel;              // items in dispatch (tile) order
-  std::vector<uint64_t> tile_base;      // tiles of rel[0..k-1]; tile_base[n] = n_tiles
+  std::vector<uint64_t> tile_base;      // records of rel[0..k-1]; tile_base[n] = n_recs
   std::vector<EmitChunk> emit_chunks;   // the emit kernel's work: every item's tiles in chunks
-  uint64_t n_tiles = 0;
+  uint64_t n_tiles = 0;                 // as the plan reports them
+  uint64_t n_recs = 0;                  // tile records, one per workgroup: at most n_tiles
   uint32_t n_src_base = 0;              // pointer table: sources, then destinations
   uint32_t n_dst_base = 0;
   std::vector<uint64_t> obj_bytes;      // per pointer-table slot: object size
@@ -754,6 +986,7 @@ struct Phase {
   DevRel* d_rel = nullptr;              // uploaded: descriptors, tile prefix, pointer table
   uint64_t* d_tile_base = nullptr;
   uint64_t* d_ptrs = nullptr;
+  EmitChunk* d_chunks = nullptr;
   DevItem* d_items = nullptr;           // built on the device
   DevTile* d_tiles = nullptr;
   unsigned char* h_staging = nullptr;   // pinned: the uploaded part, in the same layout
@@ -887,15 +1120,23 @@ uint32_t tile_reduce(const HostItem& h) {
   return (h.kind == kKindRecast && h.dst_slot >= 0) ? kRecastTileShift : 0;
 }
 
+// Whether a tile of a strided item may span 2 GiB or more of an object: its
+// rows are then addressed with 64-bit offsets.
+bool spans_far(const HostItem& h, uint32_t tile_bytes) {
+  const uint64_t rows = std::min<uint64_t>(h.rows, (uint64_t(tile_bytes) + h.row_bytes - 2) / h.row_bytes + 1);
+  const uint64_t stride = std::max({h.src_stride, h.dst_stride, h.dst2_stride});
+  return stride >= kNearBytes || rows * stride + h.row_bytes > kNearBytes;
+}
+
 void build_rel(Phase& ph, const std::vector<uint32_t>& order, uint32_t tile_bytes, bool buf_src,
                bool buf_dst, bool group_by_src, bool row_groups) {
   ph.rel.clear();
   ph.rel.reserve(order.size());
   ph.tile_base.clear();
   ph.tile_base.reserve(order.size() + 1);
-  ph.n_tiles = 0;
+  ph.n_tiles = ph.n_recs = 0;
   for (uint32_t k : order) {
-    ph.tile_base.push_back(ph.n_tiles);
+    ph.tile_base.push_back(ph.n_recs);
     const HostItem& h = ph.items[k];
     DevRel r{};
     r.src_off = h.src_off;
@@ -916,8 +1157,7 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, uint32_t tile_byte
     r.kind = h.kind | (h.esize << 8);
     if (buf_src && h.src_slot >= 0) r.kind |= kRelSrcBuf;
     if (buf_dst && h.dst_slot >= 0) r.kind |= kRelDstBuf;
-    const uint32_t reduce = tile_reduce(h);
-    r.kind |= reduce << kRelTileShiftBit;
+    if (!h.contiguous && spans_far(h, tile_bytes)) r.kind |= kRelFar;
     r.src_slot = h.src_slot;
     r.dst_slot = h.dst_slot >= 0 ? int32_t(ph.n_src_base) + h.dst_slot : -1;
     r.dst2_slot = h.dst2_slot >= 0 ? int32_t(ph.n_src_base) + h.dst2_slot : -1;
@@ -929,10 +1169,11 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, uint32_t tile_byte
     r.group_size = 1;
     r.group_index = 0;
     ph.rel.push_back(r);
-    const uint64_t item_tile = uint64_t(tile_bytes) >> reduce;
+    const uint64_t item_tile = uint64_t(tile_bytes) >> tile_reduce(h);
     ph.n_tiles += (r.total + item_tile - 1) / item_tile;
+    ph.n_recs += (r.total + tile_bytes - 1) / tile_bytes;
   }
-  ph.tile_base.push_back(ph.n_tiles);
+  ph.tile_base.push_back(ph.n_recs);
   ph.emit_chunks.clear();
   for (size_t k = 0; k < ph.rel.size(); ++k) {
     const uint64_t cnt = ph.tile_base[k + 1] - ph.tile_base[k];
@@ -955,8 +1196,7 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, uint32_t tile_byte
       const HostItem& a = ph.items[order[i - 1]];
       const HostItem& b = ph.items[order[i]];
       const Side sa = side(a), sb = side(b);
-      chain = !a.contiguous && !b.contiguous && a.kind == b.kind && tile_reduce(a) == tile_reduce(b) &&
-              a.rows == b.rows &&
+      chain = !a.contiguous && !b.contiguous && a.kind == b.kind && a.rows == b.rows &&
               a.row_bytes == b.row_bytes && sa.slot >= 0 && sa.slot == sb.slot &&
               sa.stride == sb.stride && sb.off == sa.off + sa.width;
     }
@@ -1179,6 +1419,17 @@ int setup_offsets(sr_plan* p, hipStream_t stream) {
   return SR_OK;
 }
 
+// The tile and item tables of a phase, from its descriptors and the pointer
+// table, all on the device.
+int emit_tables(sr_plan* p, Phase& ph, hipStream_t stream) {
+  const uint32_t n_chunks = uint32_t(ph.emit_chunks.size());
+  hipLaunchKernelGGL(sr_tile_emit_kernel, dim3(std::min<uint32_t>(n_chunks, 65535u)), dim3(kSetupBlock), 0, stream,
+                     ph.d_rel, ph.d_tile_base, ph.d_chunks, n_chunks, log2u(p->opt.tile_bytes), ph.d_tiles, ph.d_ptrs,
+                     p->d_offset, ph.d_items);
+  SR_HIP_TRY(hipGetLastError());
+  return SR_OK;
+}
+
 // First use of a phase: its descriptors, tile prefix and pointer table go
 // up in one copy from pinned memory, then one kernel builds the tile table
 // and binds the items to `ptrs`, stream-ordered on `stream`.  With
@@ -1202,7 +1453,7 @@ int setup_phase(sr_plan* p, Phase& ph, bool needs_offsets, const std::vector<uin
     const size_t o_ptr = carve(end, nptr * sizeof(uint64_t));
     const size_t up_end = o_ptr + nptr * sizeof(uint64_t);
     const size_t o_items = carve(end, n * sizeof(DevItem));
-    const size_t o_tiles = carve(end, ph.n_tiles * sizeof(DevTile));
+    const size_t o_tiles = carve(end, ph.n_recs * sizeof(DevTile));
     // allocations survive a failed attempt and are reused by the retry
     if (!ph.d_mem && (rc = cache.get(false, p->device, end, &ph.d_mem, &ph.d_cap)) != SR_OK) return rc;
     if (!ph.h_staging &&
@@ -1212,6 +1463,7 @@ int setup_phase(sr_plan* p, Phase& ph, bool needs_offsets, const std::vector<uin
     ph.d_rel = reinterpret_cast<DevRel*>(d + o_rel);
     ph.d_tile_base = reinterpret_cast<uint64_t*>(d + o_base);
     ph.d_ptrs = reinterpret_cast<uint64_t*>(d + o_ptr);
+    ph.d_chunks = reinterpret_cast<EmitChunk*>(d + o_chunk);
     ph.d_items = reinterpret_cast<DevItem*>(d + o_items);
     ph.d_tiles = reinterpret_cast<DevTile*>(d + o_tiles);
     ph.h_ptrs = reinterpret_cast<uint64_t*>(ph.h_staging + o_ptr);
@@ -1225,13 +1477,7 @@ int setup_phase(sr_plan* p, Phase& ph, bool needs_offsets, const std::vector<uin
       if (rc != SR_OK) return rc;
       SR_HIP_TRY(hipStreamWaitEvent(stream, p->ev_offsets, 0));
     }
-    const uint32_t shift = log2u(p->opt.tile_bytes);
-    const uint32_t n_chunks = uint32_t(ph.emit_chunks.size());
-    hipLaunchKernelGGL(sr_tile_emit_kernel, dim3(std::min<uint32_t>(n_chunks, 65535u)), dim3(kSetupBlock), 0,
-                       stream, ph.d_rel, ph.d_tile_base, reinterpret_cast<const EmitChunk*>(d + o_chunk), n_chunks,
-                       shift, ph.n_tiles, ph.interleave ? kXcds : 1u, ph.d_tiles, ph.d_ptrs, p->d_offset,
-                       ph.d_items);
-    SR_HIP_TRY(hipGetLastError());
+    if ((rc = emit_tables(p, ph, stream)) != SR_OK) return rc;
   }
   if (mark) {
     SR_HIP_TRY(hipEventRecord(ph.ev_setup, stream));
@@ -1281,6 +1527,31 @@ int check_disjoint(const Phase& ph, const std::vector<uint64_t>& ptrs) {
   return SR_OK;
 }
 
+// The copy kernel of a phase over its tables.
+int launch_copy(const sr_plan_options& opt, const Phase& ph, PhaseKind kind, const DevItem* items,
+                const DevTile* tiles, hipStream_t stream) {
+  const uint32_t n_tiles = uint32_t(ph.n_recs);
+  const uint32_t seg = ph.interleave ? (n_tiles + kXcds - 1) / kXcds : 0u;
+  const uint32_t n_pos = seg ? seg * kXcds : n_tiles;
+  uint32_t grid = n_pos;
+  if (opt.max_blocks != 0) grid = std::min(grid, opt.max_blocks);
+  grid = std::min(grid, kMaxGrid);
+  // A capped grid strides over the positions; a multiple of the segment
+  // count keeps every segment on one die.
+  if (seg && grid >= kXcds) grid -= grid % kXcds;
+  const bool nt = (opt.flags & SR_OPT_TEMPORAL) == 0;
+  typedef void (*KernelFn)(const DevItem*, const DevTile*, uint32_t, uint32_t, uint32_t, uint32_t);
+  KernelFn fn;
+  switch (kind) {
+    case kPack: fn = nt ? sr_pack_kernel<true> : sr_pack_kernel<false>; break;
+    case kUnpack: fn = nt ? sr_unpack_kernel<true> : sr_unpack_kernel<false>; break;
+    default: fn = nt ? sr_gather_kernel<true> : sr_gather_kernel<false>; break;
+  }
+  hipLaunchKernelGGL(fn, dim3(grid), dim3(kBlock), 0, stream, items, tiles, n_tiles, seg, n_pos, grid);
+  SR_HIP_TRY(hipGetLastError());
+  return SR_OK;
+}
+
 int run_phase(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>& ptrs,
               hipStream_t stream) {
   if (ph.rel.empty()) return SR_OK;
@@ -1289,7 +1560,6 @@ int run_phase(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
   if (rebind && (rc = check_disjoint(ph, ptrs)) != SR_OK) return rc;
   rc = ensure_device(p);
   if (rc != SR_OK) return rc;
-  const uint32_t n = uint32_t(ph.rel.size());
   if (!ph.ready) {
     // A phase's first use builds its tables and binds the pointers.  They
     // are the library's own memory and read no caller data: while earlier
@@ -1299,7 +1569,7 @@ int run_phase(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
     // `stream` directly, since a wait across streams costs the host more
     // than the setup kernel takes on the GPU.
     hipStream_t setup = stream;
-    if (ph.n_tiles > kInlineSetupTiles) {
+    if (ph.n_recs > kInlineSetupTiles) {
       const hipError_t busy = hipStreamQuery(stream);
       (void)hipGetLastError();   // "not ready" is an answer, not an error
       if (busy != hipSuccess && busy != hipErrorNotReady)
@@ -1321,9 +1591,7 @@ int run_phase(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
     SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_kernel, 0));
     SR_HIP_TRY(hipMemcpyAsync(ph.d_ptrs, ph.h_ptrs, ptrs.size() * sizeof(uint64_t), hipMemcpyHostToDevice,
                               stream));
-    hipLaunchKernelGGL(sr_bind_kernel, dim3((n + kSetupBlock - 1) / kSetupBlock), dim3(kSetupBlock), 0,
-                       stream, ph.d_rel, n, ph.d_ptrs, p->d_offset, ph.d_items);
-    SR_HIP_TRY(hipGetLastError());
+    if ((rc = emit_tables(p, ph, stream)) != SR_OK) return rc;
     SR_HIP_TRY(hipEventRecord(ph.ev_staging, stream));
     ph.ev_bound = ph.ev_staging;
     ph.bound = ptrs;
@@ -1333,23 +1601,7 @@ int run_phase(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
     SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_bound, 0));
   }
 
-  const uint32_t n_tiles = uint32_t(ph.n_tiles);
-  uint32_t grid = n_tiles;
-  if (p->opt.max_blocks != 0) grid = std::min(grid, p->opt.max_blocks);
-  grid = std::min(grid, kMaxGrid);
-  // A capped grid strides over the tile list; a multiple of the interleave
-  // width keeps every position on the XCD the interleave placed it for.
-  if (ph.interleave && grid < n_tiles && grid >= kXcds) grid -= grid % kXcds;
-  const bool nt = (p->opt.flags & SR_OPT_TEMPORAL) == 0;
-  typedef void (*KernelFn)(const DevItem*, const DevTile*, uint32_t);
-  KernelFn fn;
-  switch (kind) {
-    case kPack: fn = nt ? sr_pack_kernel<true> : sr_pack_kernel<false>; break;
-    case kUnpack: fn = nt ? sr_unpack_kernel<true> : sr_unpack_kernel<false>; break;
-    default: fn = nt ? sr_gather_kernel<true> : sr_gather_kernel<false>; break;
-  }
-  hipLaunchKernelGGL(fn, dim3(grid), dim3(kBlock), 0, stream, ph.d_items, ph.d_tiles, n_tiles);
-  SR_HIP_TRY(hipGetLastError());
+  if ((rc = launch_copy(p->opt, ph, kind, ph.d_items, ph.d_tiles, stream)) != SR_OK) return rc;
   SR_HIP_TRY(hipEventRecord(ph.ev_kernel, stream));
   return SR_OK;
 }
@@ -1496,6 +1748,59 @@ int sr_selftest(void) {
       if (div_apply(n, m.m, m.s1, m.s2) != n / d)
         return fail(SR_EINVAL, "selftest: %u / %u gave %u", n, d, div_apply(n, m.m, m.s1, m.s2));
     }
+  }
+  // Vectors of ragged tiles: every byte of a tile comes from its own place,
+  // no vector leaves the piece, whatever the row width and the tile's start.
+  auto check_tile = [](uint32_t width, uint32_t column, uint32_t nbytes, uint32_t piece_end) -> bool {
+    const DivMagic m = div_magic(width);
+    const RowMap rows{column, width, m.m, m.s1, m.s2};
+    std::vector<uint8_t> seen(size_t(column) + piece_end, 0);   // by byte of the rows, from the first row's start
+    auto mark = [&](uint32_t row, uint32_t col) {
+      if (col + 16 > width || uint64_t(row) * width + col + 16 > column + piece_end) return false;
+      for (uint32_t k = 0; k < 16; ++k) seen[size_t(row) * width + col + k] = 1;
+      return true;
+    };
+    for (uint32_t b = 0; b < (nbytes + 63) / 16 * 16; b += 16) {
+      const RowVec v = row_vec(rows, b, nbytes);
+      if (v.in && !mark(v.row, v.col)) return false;
+      if (v.next && !mark(v.row + 1, 0)) return false;
+    }
+    for (uint32_t b = 0; b < nbytes; ++b)
+      if (!seen[column + b]) return false;
+    return true;
+  };
+  for (uint32_t w = 16; w < 200; ++w)
+    for (uint32_t k = 0; k < 24; ++k) {
+      const uint32_t n_rows = 1 + rnd() % 40, total = w * n_rows, tile = 256;
+      const uint32_t start = rnd() % ((total + tile - 1) / tile) * tile;   // a tile of the piece
+      const uint32_t column = start % w, nbytes = std::min(tile, total - start);
+      if (!check_tile(w, column, nbytes, total - start))
+        return fail(SR_EINVAL, "selftest: rows of %u bytes, tile at %u of %u", w, start, total);
+    }
+  // Narrow vectors: each follows from the one before as a division gives it.
+  for (uint32_t w = 1; w < 700; ++w)
+    for (uint32_t k = 0; k < 8; ++k) {
+      const DivMagic m = div_magic(w);
+      const RowMap rows{rnd() % w, w, m.m, m.s1, m.s2};
+      const uint32_t step = 64u << (k & 3), ss = w + rnd() % 1000, ds = w + rnd() % 1000, hs = w + rnd() % 1000;
+      uint32_t b = rnd() % 4096;
+      RowWalk walk(rows, b, step, ss, ds, hs);
+      for (int u = 0; u < 4; ++u, b += step, walk.advance()) {
+        uint32_t row, col;
+        rows.at(b, row, col);
+        if (walk.col != col || walk.at.src != row * ss + col || walk.at.dst != row * ds + col ||
+            (w % 2 == 0 && rows.c_base % 2 == 0 && b % 2 == 0 && walk.at.half != row * hs + (col >> 1)))
+          return fail(SR_EINVAL, "selftest: walk of rows of %u bytes, step %u", w, step);
+      }
+    }
+  for (uint32_t n = 16; n < 300; ++n) {
+    std::vector<uint8_t> seen(n, 0);
+    for (uint32_t b = 0; b < n + 64; b += 16) {
+      const uint32_t off = contiguous_vec(b, n);
+      if (b >= n ? off < n : off + 16 > n) return fail(SR_EINVAL, "selftest: vector %u of %u contiguous bytes", b, n);
+      if (b < n) std::fill_n(seen.begin() + off, 16, 1);
+    }
+    if (std::count(seen.begin(), seen.end(), 1) != n) return fail(SR_EINVAL, "selftest: %u contiguous bytes", n);
   }
   return SR_OK;
 }
@@ -1771,7 +2076,8 @@ int sr_plan_create(const sr_tensor* src_tensors, int32_t n_src, const sr_tensor*
       delete p;
       return fail(SR_EINVAL, "plan has too many tiles; raise tile_bytes");
     }
-    ph->interleave = !(opt.flags & SR_OPT_NO_XCD_INTERLEAVE) && ph->n_tiles >= 2 * uint64_t(kXcds);
+    ph->interleave = !(opt.flags & SR_OPT_NO_XCD_INTERLEAVE) && ph->n_recs >= 2 * uint64_t(kXcds) &&
+                     ph->n_recs <= UINT32_MAX - kXcds;
   }
   // Per-peer piece lists (piece order) and payloads, from which the device
   // recomputes the buffer offsets.
@@ -1985,23 +2291,12 @@ int sr_gather_noalloc(const sr_plan* plan, const void* const* src_ptrs, void* co
                             stream));
   SR_HIP_TRY(hipMemcpyAsync(d_ptrs, ptrs.data(), ptrs.size() * sizeof(uint64_t), hipMemcpyHostToDevice,
                             stream));
-  const uint32_t shift = log2u(plan->opt.tile_bytes);
   // gather items read no buffer offsets (no side is a peer buffer)
   hipLaunchKernelGGL(sr_tile_emit_kernel, dim3(std::min<uint32_t>(n_chunks, 65535u)), dim3(kSetupBlock), 0,
-                     stream, d_rel, d_base, d_chunks, n_chunks, shift, ph.n_tiles, ph.interleave ? kXcds : 1u,
-                     d_tiles, d_ptrs, static_cast<const uint64_t*>(nullptr), d_items);
+                     stream, d_rel, d_base, d_chunks, n_chunks, log2u(plan->opt.tile_bytes), d_tiles, d_ptrs,
+                     static_cast<const uint64_t*>(nullptr), d_items);
   SR_HIP_TRY(hipGetLastError());
-
-  const uint32_t n_tiles = uint32_t(ph.n_tiles);
-  uint32_t grid = n_tiles;
-  if (plan->opt.max_blocks != 0) grid = std::min(grid, plan->opt.max_blocks);
-  grid = std::min(grid, kMaxGrid);
-  if (ph.interleave && grid < n_tiles && grid >= kXcds) grid -= grid % kXcds;
-  const bool nt = (plan->opt.flags & SR_OPT_TEMPORAL) == 0;
-  hipLaunchKernelGGL(nt ? sr_gather_kernel<true> : sr_gather_kernel<false>, dim3(grid), dim3(kBlock), 0,
-                     stream, d_items, d_tiles, n_tiles);
-  SR_HIP_TRY(hipGetLastError());
-  return SR_OK;
+  return launch_copy(plan->opt, ph, kGather, d_items, d_tiles, stream);
 }
 
 void sr_plan_destroy(sr_plan* plan) {

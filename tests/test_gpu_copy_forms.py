@@ -1,0 +1,161 @@
+"""The copy kernels' forms at the sizes where they change: rows narrower and
+wider than a vector, multiples of 16 bytes or not, merged and split bands of
+columns, dense and strided destinations, misaligned objects, tiles that start
+and end in the middle of a row, a last vector that is not whole, RECAST and
+ZERO pieces, rows 2 GiB apart.  Every case is byte movement or one rounding:
+exact against torch, with the bytes around each destination untouched."""
+import ctypes
+
+import pytest
+import torch
+
+from suika_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+DT = {"u8": (_lib.SR_DT_U8, torch.uint8), "bf16": (_lib.SR_DT_BF16, torch.bfloat16),
+      "f32": (_lib.SR_DT_F32, torch.float32), "f64": (_lib.SR_DT_F64, torch.float64)}
+COPY, RECAST, ZERO = _lib.SR_PIECE_COPY, _lib.SR_PIECE_RECAST, _lib.SR_PIECE_ZERO
+GUARD = 64       # elements around each object
+POISON = 0xA7
+
+
+class Obj:
+    """A [rows, cols] object `shift` elements into a guarded allocation."""
+
+    def __init__(self, rows, cols, dt, shift=0, seed=None):
+        self.rows, self.cols, self.dt = rows, cols, dt
+        tdt = DT[dt][1]
+        self.buf = torch.empty(rows * cols + 2 * GUARD, dtype=tdt, device="cuda")
+        self.bytes = self.buf.view(torch.uint8)
+        self.at = GUARD + shift
+        self.es = self.buf.element_size()
+        if seed is None:
+            self.bytes.fill_(POISON)
+        else:
+            g = torch.Generator("cuda").manual_seed(seed)
+            if tdt.is_floating_point:
+                self.buf.copy_(torch.randn(self.buf.shape, generator=g, device="cuda"))
+            else:
+                self.buf.copy_(torch.randint(0, 256, self.buf.shape, generator=g, device="cuda"))
+        self.t = self.buf[self.at:self.at + rows * cols].view(rows, cols)
+
+    def check(self, want, what):
+        got = self.t.contiguous().view(torch.uint8)
+        assert torch.equal(got, want.contiguous().view(torch.uint8)), what
+        lo, hi = self.at * self.es, (self.at + self.rows * self.cols) * self.es
+        assert bool((self.bytes[:lo] == POISON).all()) and bool((self.bytes[hi:] == POISON).all()), f"{what}: guard"
+
+
+def _gather(src, dst, pieces, tile_bytes=0, flags=0, noalloc=False):
+    L = _lib.lib()
+    S = (_lib.SrTensor * max(1, len(src)))(*[_lib.SrTensor(o.rows, o.cols, DT[o.dt][0], 0) for o in src])
+    D = (_lib.SrTensor * len(dst))(*[_lib.SrTensor(o.rows, o.cols, DT[o.dt][0], 0) for o in dst])
+    P = (_lib.SrPiece * len(pieces))(*[_lib.SrPiece(*p) for p in pieces])
+    opt = _lib.SrPlanOptions(tile_bytes, 0, flags, 0)
+    h = ctypes.c_void_p()
+    _lib.check(L.sr_plan_create(S, len(src), D, len(dst), 1, P, len(pieces), ctypes.byref(opt), ctypes.byref(h)), "plan")
+    try:
+        vp = ctypes.c_void_p
+        sp = (vp * max(1, len(src)))(*[o.t.data_ptr() for o in src])
+        dp = (vp * len(dst))(*[o.t.data_ptr() for o in dst])
+        call = L.sr_gather_noalloc if noalloc else L.sr_gather
+        _lib.check(call(h, sp, dp, vp(torch.cuda.current_stream().cuda_stream)), "gather")
+        torch.cuda.synchronize()
+    finally:
+        L.sr_plan_destroy(h)
+
+
+def copy(si, di, rows, cols, sc=0, dc=0, sr=0, dr=0):
+    return (COPY, 0, si, di, -1, 0, rows, cols, sr, sc, dr, dc)
+
+
+# bytes per row: below a vector, around 16, around the widths where short rows
+# end (64, 384, 400, 512), around a wave's and a tile's vectors
+ROWS = [1, 2, 3, 6, 8, 12, 15, 16, 17, 24, 33, 48, 63, 64, 66, 96, 128, 192, 382, 384, 398, 400, 402, 510, 512, 514,
+        1022, 1024, 1028, 2730, 5460, 16382, 16384, 16400]
+
+
+@pytest.mark.parametrize("tile_bytes", [0, 4096, 1 << 16])
+@pytest.mark.parametrize("dt", sorted(DT))
+def test_bands_of_columns(dt, tile_bytes):
+    """Two bands merged side by side and split apart, at every row width that
+    is whole elements."""
+    es = torch.empty(0, dtype=DT[dt][1]).element_size()
+    for k, width in enumerate(w for w in ROWS if w % es == 0):
+        c = width // es
+        rows = max(3, min(5000, 150000 // width))
+        print(f"[copy forms] {dt} rows of {width} B, tile {tile_bytes}", flush=True)
+        a, b = Obj(rows, c, dt, seed=3 * k), Obj(rows, c, dt, seed=3 * k + 1)
+        d = Obj(rows, 2 * c, dt)
+        _gather([a, b], [d], [copy(0, 0, rows, c), copy(1, 0, rows, c, dc=c)], tile_bytes)
+        d.check(torch.cat([a.t, b.t], 1), f"merge {width}")
+        s = Obj(rows, 2 * c, dt, seed=3 * k + 2)
+        x, y = Obj(rows, c, dt), Obj(rows, c, dt)
+        _gather([s], [x, y], [copy(0, 0, rows, c), copy(0, 1, rows, c, sc=c)], tile_bytes, noalloc=tile_bytes == 4096)
+        x.check(s.t[:, :c], f"split {width}")
+        y.check(s.t[:, c:], f"split {width}")
+
+
+@pytest.mark.parametrize("shift", [(0, 0), (1, 0), (0, 1), (3, 1)])
+@pytest.mark.parametrize("dt", sorted(DT))
+def test_contiguous_pieces_at_any_alignment(dt, shift):
+    es = torch.empty(0, dtype=DT[dt][1]).element_size()
+    sizes = {1, 2, 3, 15, 16, 17, 16384 // es - 1, 16384 // es, 16384 // es + 1, 16384 // es + 3, 40000 // es + 1,
+             (8 * 16384 + 5 * es) // es}
+    for n in sorted(sizes):
+        print(f"[copy forms] {dt} contiguous {n}, shift {shift}", flush=True)
+        a, d = Obj(1, n, dt, shift[0], seed=n), Obj(1, n, dt, shift[1])
+        _gather([a], [d], [copy(0, 0, 1, n)])
+        d.check(a.t, n)
+        z = Obj(1, n, dt, shift[1])
+        _gather([], [z], [(ZERO, 0, -1, 0, -1, 0, 1, n, 0, 0, 0, 0)])
+        z.check(torch.zeros_like(z.t), n)
+
+
+@pytest.mark.parametrize("flags", [0, _lib.SR_OPT_TEMPORAL | _lib.SR_OPT_NO_XCD_INTERLEAVE])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_recast_and_zero_rows(shift, flags):
+    """RECAST bands with and without the f32 copy, beside ZERO bands."""
+    for c in (1, 3, 4, 5, 16, 20, 32, 33, 64, 96, 100, 257, 683, 4096, 4100):
+        rows = max(3, min(3000, 40000 // c))
+        print(f"[copy forms] recast rows of {c}, shift {shift}", flush=True)
+        a, b = Obj(rows, c, "f32", shift, seed=c), Obj(rows, 2 * c, "f32", seed=c + 1)
+        d, h = Obj(rows, 3 * c, "f32", shift), Obj(rows, 3 * c, "bf16", shift)
+        x, y = Obj(rows, c, "f32"), Obj(rows, c, "bf16")
+        n = Obj(rows, 2 * c, "bf16", shift)
+        _gather([a, b], [d, h, x, y, n],
+                [(RECAST, 0, 0, 0, 1, 0, rows, c, 0, 0, 0, 0), (RECAST, 0, 1, 0, 1, 0, rows, c, 0, c, 0, c),
+                 (ZERO, 0, -1, 0, -1, 0, rows, c, 0, 0, 0, 2 * c), (ZERO, 0, -1, 1, -1, 0, rows, c, 0, 0, 0, 2 * c),
+                 (RECAST, 0, 1, 2, 3, 0, rows, c, 0, 0, 0, 0),
+                 (RECAST, 0, 0, -1, 4, 0, rows, c, 0, 0, 0, 0), (RECAST, 0, 1, -1, 4, 0, rows, c, 0, 0, 0, c)],
+                flags=flags)
+        want = torch.cat([a.t, b.t[:, c:], torch.zeros_like(a.t)], 1)
+        d.check(want, c)
+        h.check(want.to(torch.bfloat16), c)
+        x.check(b.t[:, :c], c)
+        y.check(b.t[:, :c].to(torch.bfloat16), c)
+        n.check(torch.cat([a.t, b.t[:, :c]], 1).to(torch.bfloat16), c)
+
+
+def test_rows_two_gib_apart():
+    """Rows so long that a tile's rows span 2 GiB: 64-bit offsets, beside a
+    band of the same rows that is near enough within a smaller tile."""
+    rows, cols = 3, 900_000_001
+    print("[copy forms] rows 0.9 GB apart", flush=True)
+    src = torch.zeros(rows * cols, dtype=torch.uint8, device="cuda").view(rows, cols)
+    bands = {0: 7, 1000: 16, 5000: 200, cols - 40001: 40001}
+    g = torch.Generator("cuda").manual_seed(1)
+    for at, w in bands.items():
+        src[:, at:at + w] = torch.randint(0, 256, (rows, w), generator=g, device="cuda", dtype=torch.uint8)
+
+    class Whole:
+        pass
+    s = Whole()
+    s.rows, s.cols, s.dt, s.t = rows, cols, "u8", src
+    dst = [Obj(rows, w, "u8") for w in bands.values()]
+    _gather([s], dst, [copy(0, k, rows, w, sc=at) for k, (at, w) in enumerate(bands.items())])
+    for d, (at, w) in zip(dst, bands.items()):
+        d.check(src[:, at:at + w], f"band at {at}")
+    del s, src
+    torch.cuda.empty_cache()
