@@ -243,7 +243,7 @@ int sr_gather(sr_plan* plan, const void* const* src_ptrs, void* const* dst_ptrs,
  *   - The descriptors and pointers are uploaded from pageable host memory at
  *     every call, which HIP performs synchronously: the call blocks the host
  *     until the work queued on `stream` before it has finished and the tables
- *     are on the device; the tile, bind and copy kernels then run
+ *     are on the device; the table and copy kernels then run
  *     asynchronously.  For the same reason the call cannot be recorded into a
  *     HIP graph: on a stream that is capturing it returns SR_EINVAL and does
  *     nothing.
