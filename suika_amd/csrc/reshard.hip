@@ -626,7 +626,8 @@ __device__ __forceinline__ void far_tile(const DevItem& it, const DevTile& t, ui
 // workgroup's; `stride` is the grid.
 template <bool NT>
 __device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, const DevTile* __restrict__ tiles,
-                                           uint32_t n_tiles, uint32_t seg, uint32_t n_pos, uint32_t stride) {
+                                           uint32_t n_tiles, uint32_t seg, uint32_t n_pos, uint32_t stride,
+                                           uint32_t n_ahead) {
   uint32_t p = blockIdx.x;
   do {
     const uint32_t i = seg ? (p % kXcds) * seg + p / kXcds : p;
@@ -636,7 +637,7 @@ __device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, co
       // be computed for all paths before the loop, and held
       uint32_t lane = threadIdx.x;
       asm volatile("" : "+v"(lane));
-      const Ahead ahead{tiles, i, n_tiles, lane};
+      const Ahead ahead{tiles, i, n_ahead, lane};
       const uint32_t op = t.info >> kTileOpBit, nbytes = t.info & kTileBytesMask;
       constexpr Policy kWhole = NT ? kThrough : kCached, kPartial = NT ? kStream : kCached;
       const Region none = region(0, 0);
@@ -690,8 +691,8 @@ __device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, co
   template <bool NT>                                                                                              \
   __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(8))) void NAME(    \
       const DevItem* __restrict__ items, const DevTile* __restrict__ tiles, uint32_t n_tiles, uint32_t seg,       \
-      uint32_t n_pos, uint32_t stride) {                                                                          \
-    exec_tiles<NT>(items, tiles, n_tiles, seg, n_pos, stride);                                                    \
+      uint32_t n_pos, uint32_t stride, uint32_t n_ahead) {                                                        \
+    exec_tiles<NT>(items, tiles, n_tiles, seg, n_pos, stride, n_ahead);                                           \
   }
 SR_COPY_KERNEL(sr_pack_kernel)
 SR_COPY_KERNEL(sr_unpack_kernel)
@@ -775,6 +776,26 @@ constexpr uint32_t kEmitTiles = 4096;
 // of GPU time, less than a wait across streams costs the host.
 constexpr uint64_t kInlineSetupTiles = 65536;
 
+// Phases of at most this many tiles have their tables written by the host
+// and read from its memory at the first launch on new pointers, which saves
+// the emit kernel.  Above, the tiles' reads over the host link and the host's
+// writes cost more.  A call with new pointers, us, emit / host tables (f32
+// rows of 8 KiB split off): 8 tiles 19.2 / 8.0, 512 20.8 / 9.6, 1024 21.9 /
+// 13.0, 2048 26.7 / 21.3, 4096 37.1 / 38.7.  Launches that repeat the pointers
+// read device memory, as 2048 tiles take 21.4 from the host's and 14.4 from
+// the device's.
+constexpr uint64_t kHostTableTiles = 2048;
+
+// `vectors` 16-byte vectors of a table from pinned host memory to the device:
+// bound by the host link's latency, one read per lane in flight.
+__global__ __launch_bounds__(kSetupBlock) void sr_table_copy_kernel(const unsigned char* __restrict__ from,
+                                                                    unsigned char* __restrict__ to,
+                                                                    uint32_t vectors) {
+  typedef VecOf<16>::type V;
+  const uint32_t i = blockIdx.x * kSetupBlock + threadIdx.x;
+  if (i < vectors) reinterpret_cast<V*>(to)[i] = reinterpret_cast<const V*>(from)[i];
+}
+
 // An empty kernel: launching it loads the library's GPU code (sr_prepare).
 __global__ void sr_prepare_kernel() {}
 
@@ -842,7 +863,7 @@ constexpr uint32_t kMergeBelow = 512, kMergeZeroBelow = 384;
 // the phase's pointer table (source objects, then destination objects),
 // and `offset`, the per-piece buffer offsets from sr_offsets_kernel; the
 // vector and the op of its tiles.
-__device__ __forceinline__ DevItem bind_item(const DevRel& h, const uint64_t* __restrict__ ptrs,
+__host__ __device__ __forceinline__ DevItem bind_item(const DevRel& h, const uint64_t* __restrict__ ptrs,
                                              const uint64_t* __restrict__ offset, uint32_t& op) {
   const uint32_t kind = h.kind & 0xffu;
   const bool contiguous = h.row_bytes == 0;
@@ -895,6 +916,30 @@ __device__ __forceinline__ DevItem bind_item(const DevRel& h, const uint64_t* __
   return d;
 }
 
+// Tile `j` of item `k` of `total` source bytes, bound as `item`.
+__host__ __device__ __forceinline__ DevTile tile_record(const DevItem& item, uint32_t k, uint32_t op, uint64_t total,
+                                                        uint32_t tile_shift, uint64_t j) {
+  const uint32_t width = item.row_bytes;
+  uint64_t start = j << tile_shift;
+  uint64_t n = total - start < (uint64_t(1) << tile_shift) ? total - start : (uint64_t(1) << tile_shift);
+  if (width == 0 && total >= 16 && n < 16) {   // a whole vector, from the tile before
+    start -= 16 - n;
+    n = 16;
+  }
+  DevTile t;
+  t.item = k;
+  t.info = op << kTileOpBit | uint32_t(n);
+  if (width == 0) {
+    t.src = item.src + start;
+    t.dst = item.dst ? item.dst + start : 0;
+  } else {
+    const uint64_t row = start / width;
+    t.src = row;
+    t.dst = start - row * width;
+  }
+  return t;
+}
+
 // One workgroup per emit chunk -- up to kEmitTiles consecutive tiles of one
 // item (chunks[c] = {item, chunk index}; every item has at least one) --
 // writes those tiles' records, in list order (tile_base[k] = tiles of items
@@ -909,7 +954,6 @@ __global__ __launch_bounds__(kSetupBlock) void sr_tile_emit_kernel(
     const uint32_t k = chunks[c].item;
     const uint64_t j0 = uint64_t(chunks[c].chunk) * kEmitTiles;
     const uint64_t total = rel[k].total;
-    const uint32_t width = rel[k].row_bytes;
     const uint64_t cnt = tile_base[k + 1] - tile_base[k];
     // Items of a group have equal tile counts; tile j of member m goes to
     // group_start + j*M + m, so the members' tiles over the same rows are
@@ -920,27 +964,9 @@ __global__ __launch_bounds__(kSetupBlock) void sr_tile_emit_kernel(
     uint32_t op;
     const DevItem item = bind_item(rel[k], ptrs, offset, op);
     if (j0 == 0 && threadIdx.x == 0) items[k] = item;
-    const uint32_t info = op << kTileOpBit;
     const uint64_t j1 = cnt < j0 + kEmitTiles ? cnt : j0 + kEmitTiles;
     for (uint64_t j = j0 + threadIdx.x; j < j1; j += kSetupBlock) {
-      uint64_t start = j << tile_shift;
-      uint64_t n = total - start < (uint64_t(1) << tile_shift) ? total - start : (uint64_t(1) << tile_shift);
-      if (width == 0 && total >= 16 && n < 16) {   // a whole vector, from the tile before
-        start -= 16 - n;
-        n = 16;
-      }
-      DevTile t;
-      t.item = k;
-      t.info = info | uint32_t(n);
-      if (width == 0) {
-        t.src = item.src + start;
-        t.dst = item.dst ? item.dst + start : 0;
-      } else {
-        const uint64_t row = start / width;
-        t.src = row;
-        t.dst = start - row * width;
-      }
-      tiles[b + j * gsize] = t;
+      tiles[b + j * gsize] = tile_record(item, k, op, total, tile_shift, j);
     }
   }
 }
@@ -1001,6 +1027,10 @@ struct Phase {
   hipEvent_t ev_staging = nullptr;      // a later bind done (its reads of h_staging too)
   hipEvent_t ev_kernel = nullptr;       // last kernel reading d_items
   hipEvent_t ev_bound = nullptr;        // the latest bind: ev_setup or ev_staging (not owned)
+  // small phases (kHostTableTiles): two pinned tables in h_staging, written in turn
+  int slot = 0;
+  hipEvent_t ev_slot[2] = {};           // last kernel reading the table
+  bool on_device = false;               // the tables are in d_mem too
 };
 
 }  // namespace
@@ -1532,7 +1562,7 @@ int check_disjoint(const Phase& ph, const std::vector<uint64_t>& ptrs) {
 
 // The copy kernel of a phase over its tables.
 int launch_copy(const sr_plan_options& opt, const Phase& ph, PhaseKind kind, const DevItem* items,
-                const DevTile* tiles, hipStream_t stream) {
+                const DevTile* tiles, bool read_ahead, hipStream_t stream) {
   const uint32_t n_tiles = uint32_t(ph.n_recs);
   const uint32_t seg = ph.interleave ? (n_tiles + kXcds - 1) / kXcds : 0u;
   const uint32_t n_pos = seg ? seg * kXcds : n_tiles;
@@ -1543,15 +1573,79 @@ int launch_copy(const sr_plan_options& opt, const Phase& ph, PhaseKind kind, con
   // count keeps every segment on one die.
   if (seg && grid >= kXcds) grid -= grid % kXcds;
   const bool nt = (opt.flags & SR_OPT_TEMPORAL) == 0;
-  typedef void (*KernelFn)(const DevItem*, const DevTile*, uint32_t, uint32_t, uint32_t, uint32_t);
+  typedef void (*KernelFn)(const DevItem*, const DevTile*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t);
   KernelFn fn;
   switch (kind) {
     case kPack: fn = nt ? sr_pack_kernel<true> : sr_pack_kernel<false>; break;
     case kUnpack: fn = nt ? sr_unpack_kernel<true> : sr_unpack_kernel<false>; break;
     default: fn = nt ? sr_gather_kernel<true> : sr_gather_kernel<false>; break;
   }
-  hipLaunchKernelGGL(fn, dim3(grid), dim3(kBlock), 0, stream, items, tiles, n_tiles, seg, n_pos, grid);
+  hipLaunchKernelGGL(fn, dim3(grid), dim3(kBlock), 0, stream, items, tiles, n_tiles, seg, n_pos, grid,
+                     read_ahead ? n_tiles : 0u);
   SR_HIP_TRY(hipGetLastError());
+  return SR_OK;
+}
+
+// The launch of a phase of at most kHostTableTiles tiles.  On new pointers the
+// host writes the items and tile records, bound, to pinned memory and the copy
+// kernel reads them there.  A second launch with the same pointers copies the
+// tables to the device first and reads them there, as the ones after it do.
+// Other pointers go to the other of two pinned tables, so the host waits only
+// for a launch two bindings ago.
+int run_small(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>& ptrs, bool rebind,
+              hipStream_t stream) {
+  TableCache& cache = table_cache();
+  const size_t n = ph.rel.size();
+  size_t end = 0;
+  const size_t o_items = carve(end, n * sizeof(DevItem));
+  const size_t o_tiles = carve(end, ph.n_recs * sizeof(DevTile));
+  const size_t half = carve(end, 0);
+  int rc;
+  if (!ph.h_staging &&
+      (rc = cache.get(true, p->device, 2 * half, reinterpret_cast<void**>(&ph.h_staging), &ph.h_cap)) != SR_OK)
+    return rc;
+  const int slot = rebind ? ph.slot ^ 1 : ph.slot;
+  unsigned char* table = ph.h_staging + slot * half;
+  if (rebind) {
+    if (ph.ev_slot[slot]) SR_HIP_TRY(hipEventSynchronize(ph.ev_slot[slot]));
+    else if ((rc = cache.get_event(p->device, &ph.ev_slot[slot])) != SR_OK) return rc;
+    ph.bound_valid = ph.on_device = false;
+    DevItem* items = reinterpret_cast<DevItem*>(table + o_items);
+    DevTile* tiles = reinterpret_cast<DevTile*>(table + o_tiles);
+    const uint32_t tile_shift = log2u(p->opt.tile_bytes);
+    for (uint32_t k = 0; k < n; ++k) {
+      const DevRel& h = ph.rel[k];
+      uint32_t op;
+      const DevItem item = bind_item(h, ptrs.data(), p->piece_offset.data(), op);
+      items[k] = item;
+      const uint64_t cnt = ph.tile_base[k + 1] - ph.tile_base[k];
+      DevTile* t = tiles + (ph.tile_base[k] - h.group_index * cnt + h.group_index);
+      for (uint64_t j = 0; j < cnt; ++j) t[j * h.group_size] = tile_record(item, k, op, h.total, tile_shift, j);
+    }
+    ph.slot = slot;
+    ph.bound = ptrs;
+    ph.bound_valid = true;
+  }
+  if (!rebind && !ph.on_device) {
+    if (!ph.ev_setup && (rc = cache.get_event(p->device, &ph.ev_setup)) != SR_OK) return rc;
+    if (!ph.ev_kernel && (rc = cache.get_event(p->device, &ph.ev_kernel)) != SR_OK) return rc;
+    if (!ph.d_mem && (rc = cache.get(false, p->device, half, &ph.d_mem, &ph.d_cap)) != SR_OK) return rc;
+    SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_kernel, 0));   // the last reader of the device's tables
+    const uint32_t vectors = uint32_t(half / 16);
+    hipLaunchKernelGGL(sr_table_copy_kernel, dim3((vectors + kSetupBlock - 1) / kSetupBlock), dim3(kSetupBlock), 0,
+                       stream, table, static_cast<unsigned char*>(ph.d_mem), vectors);
+    SR_HIP_TRY(hipGetLastError());
+    SR_HIP_TRY(hipEventRecord(ph.ev_setup, stream));
+    SR_HIP_TRY(hipEventRecord(ph.ev_slot[slot], stream));
+    ph.on_device = true;
+  } else if (ph.on_device) {
+    SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_setup, 0));
+  }
+  if (ph.on_device) table = static_cast<unsigned char*>(ph.d_mem);
+  rc = launch_copy(p->opt, ph, kind, reinterpret_cast<DevItem*>(table + o_items),
+                   reinterpret_cast<DevTile*>(table + o_tiles), ph.on_device, stream);
+  if (rc != SR_OK) return rc;
+  SR_HIP_TRY(hipEventRecord(ph.on_device ? ph.ev_kernel : ph.ev_slot[slot], stream));
   return SR_OK;
 }
 
@@ -1563,6 +1657,14 @@ int run_phase(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
   if (rebind && (rc = check_disjoint(ph, ptrs)) != SR_OK) return rc;
   rc = ensure_device(p);
   if (rc != SR_OK) return rc;
+  if (ph.n_recs <= kHostTableTiles && !ph.ready) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();   // the launch reports it
+    if (cap == hipStreamCaptureStatusNone) return run_small(p, ph, kind, ptrs, rebind, stream);
+    // A graph would replay reads of tables that the host writes again; a
+    // phase whose first use is captured keeps the device tables below.
+    if (ph.h_staging) return fail(SR_EHIP, "a plan that has run before cannot be captured into a graph");
+  }
   if (!ph.ready) {
     // A phase's first use builds its tables and binds the pointers.  They
     // are the library's own memory and read no caller data: while earlier
@@ -1602,7 +1704,7 @@ int run_phase(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
     SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_bound, 0));
   }
 
-  if ((rc = launch_copy(p->opt, ph, kind, ph.d_items, ph.d_tiles, stream)) != SR_OK) return rc;
+  if ((rc = launch_copy(p->opt, ph, kind, ph.d_items, ph.d_tiles, true, stream)) != SR_OK) return rc;
   SR_HIP_TRY(hipEventRecord(ph.ev_kernel, stream));
   return SR_OK;
 }
@@ -1612,11 +1714,11 @@ int run_phase(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
 // be destroyed right after an asynchronous call.
 void free_phase(Phase& ph, int device) {
   TableCache& cache = table_cache();
-  for (hipEvent_t ev : {ph.ev_kernel, ph.ev_staging, ph.ev_setup})
+  for (hipEvent_t ev : {ph.ev_kernel, ph.ev_staging, ph.ev_setup, ph.ev_slot[0], ph.ev_slot[1]})
     if (ev) (void)hipEventSynchronize(ev);
   cache.put(false, device, ph.d_mem, ph.d_cap);
   cache.put(true, device, ph.h_staging, ph.h_cap);
-  for (hipEvent_t ev : {ph.ev_setup, ph.ev_staging, ph.ev_kernel}) cache.put_event(device, ev);
+  for (hipEvent_t ev : {ph.ev_setup, ph.ev_staging, ph.ev_kernel, ph.ev_slot[0], ph.ev_slot[1]}) cache.put_event(device, ev);
   ph = Phase();
 }
 
@@ -2301,7 +2403,7 @@ int sr_gather_noalloc(const sr_plan* plan, const void* const* src_ptrs, void* co
                      stream, d_rel, d_base, d_chunks, n_chunks, log2u(plan->opt.tile_bytes), d_tiles, d_ptrs,
                      static_cast<const uint64_t*>(nullptr), d_items);
   SR_HIP_TRY(hipGetLastError());
-  return launch_copy(plan->opt, ph, kGather, d_items, d_tiles, stream);
+  return launch_copy(plan->opt, ph, kGather, d_items, d_tiles, true, stream);
 }
 
 void sr_plan_destroy(sr_plan* plan) {

@@ -1,0 +1,131 @@
+"""Small phases: tables written by the host at the first launch on new
+pointers, device tables from the second.  Around the tile count where the
+other route begins, both give torch's bytes, also where bindings take turns
+without a host synchronisation.  All exact."""
+import ctypes
+
+import pytest
+import torch
+
+from suika_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+LIMIT = 2048     # tiles up to which the host writes the tables
+TILE = 4096
+vp = ctypes.c_void_p
+
+
+class Plan:
+    """[rows, cols] f32 source: columns split off as f32, the rest recast into
+    f32 + bf16, zero-filled rows, and whole rows up to `tiles` tiles."""
+
+    def __init__(self, tiles, cols=333, rows=40, split=100):
+        self.rows, self.cols, self.split = rows, cols, split
+        piece = _lib.SrPiece
+        small = -(-rows * split * 4 // TILE) + -(-rows * (cols - split) * 4 // TILE) + 1
+        self.fill = (tiles - small) * TILE // 4
+        assert self.fill > 0
+        f32, bf16 = _lib.SR_DT_F32, _lib.SR_DT_BF16
+        T = _lib.SrTensor
+        S = (T * 2)(T(rows, cols, f32, 0), T(1, self.fill, f32, 0))
+        D = (T * 4)(T(rows + 3, split, f32, 0), T(rows, cols - split, f32, 0), T(rows, cols - split, bf16, 0),
+                    T(1, self.fill, f32, 0))
+        P = [piece(_lib.SR_PIECE_COPY, 0, 0, 0, -1, 0, rows, split, 0, 0, 0, 0),
+             piece(_lib.SR_PIECE_ZERO, 0, -1, 0, -1, 0, 3, split, 0, 0, rows, 0),
+             piece(_lib.SR_PIECE_RECAST, 0, 0, 1, 2, 0, rows, cols - split, 0, split, 0, 0),
+             piece(_lib.SR_PIECE_COPY, 0, 1, 3, -1, 0, 1, self.fill, 0, 0, 0, 0)]
+        opt = _lib.SrPlanOptions(TILE, 0, 0, 0)
+        self.h = vp()
+        self.L = _lib.lib()
+        _lib.check(self.L.sr_plan_create(S, 2, D, 4, 1, (piece * 4)(*P), 4, ctypes.byref(opt), ctypes.byref(self.h)),
+                   "plan")
+        n = ctypes.c_uint64()
+        _lib.check(self.L.sr_plan_peer_bytes(self.h, 0, ctypes.byref(n)), "peer bytes")
+        self.peer_bytes = n.value
+
+    def src(self, seed):
+        g = torch.Generator("cuda").manual_seed(seed)
+        return [torch.randn(self.rows, self.cols, generator=g, device="cuda"),
+                torch.randn(1, self.fill, generator=g, device="cuda")]
+
+    def dst(self):
+        w = self.cols - self.split
+        return [torch.full((self.rows + 3, self.split), 7.0, device="cuda"),
+                torch.full((self.rows, w), 7.0, device="cuda"),
+                torch.full((self.rows, w), 7.0, device="cuda", dtype=torch.bfloat16),
+                torch.full((1, self.fill), 7.0, device="cuda")]
+
+    def gather(self, src, dst):
+        self._call(self.L.sr_gather, src, dst)
+
+    def _call(self, fn, a, b):
+        A, B = (vp * len(a))(*[t.data_ptr() for t in a]), (vp * len(b))(*[t.data_ptr() for t in b])
+        _lib.check(fn(self.h, A, B, vp(torch.cuda.current_stream().cuda_stream)), "call")
+
+    def exchange(self, src, buf, dst):
+        self._call(self.L.sr_pack, src, [buf])
+        self._call(self.L.sr_unpack, [buf], dst)
+
+    def check(self, src, dst):
+        want = [torch.cat([src[0][:, :self.split], src[0].new_zeros(3, self.split)]), src[0][:, self.split:],
+                src[0][:, self.split:].to(torch.bfloat16), src[1]]
+        for k, (a, b) in enumerate(zip(dst, want)):
+            assert torch.equal(a, b), f"destination {k}"
+
+    def close(self):
+        torch.cuda.synchronize()
+        self.L.sr_plan_destroy(self.h)
+
+
+@pytest.mark.parametrize("cols,split", [(333, 100), (336, 96), (40, 3)])
+@pytest.mark.parametrize("tiles", [64, LIMIT - 1, LIMIT, LIMIT + 1])
+def test_bindings_in_turn(tiles, cols, split):
+    print(f"[gpu host tables] {tiles} tiles, {cols} columns at {split}", flush=True)
+    p = Plan(tiles, cols=cols, split=split)
+    try:
+        srcs, dsts = [p.src(i) for i in range(3)], [p.dst() for _ in range(3)]
+        for i in (0, 1, 2, 1, 1, 1, 0, 2, 2):   # first, second and third launches of a binding, and returns to it
+            for t in dsts[i]:
+                t.fill_(7)
+            p.gather(srcs[i], dsts[i])
+        for s, d in zip(srcs, dsts):
+            p.check(s, d)
+        bufs = [torch.empty(p.peer_bytes, dtype=torch.uint8, device="cuda") for _ in range(2)]
+        for i in (0, 1, 1, 0):
+            for t in dsts[i]:
+                t.fill_(7)
+            p.exchange(srcs[i], bufs[i], dsts[i])
+        for i in range(2):
+            p.check(srcs[i], dsts[i])
+    finally:
+        p.close()
+
+
+def test_graph_capture_stays_refused():
+    """A plan that has run is refused on a capturing stream before any device
+    work: the capture stays valid, and so does the plan."""
+    print("[gpu host tables] capture refused", flush=True)
+    p = Plan(64)
+    try:
+        src, dst = p.src(0), p.dst()
+        mark = torch.zeros(64, device="cuda")
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(2):   # bound by the host, then on the device
+                p.gather(src, dst)
+                stream.synchronize()
+                g = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(g, stream=stream):
+                    mark.add_(1.0)
+                    with pytest.raises(_lib.ReshardError, match="cannot be captured"):
+                        p.gather(src, dst)
+                for _ in range(2):
+                    g.replay()
+            src[0].add_(1.0)
+            p.gather(src, dst)
+            stream.synchronize()
+        p.check(src, dst)
+        assert torch.equal(mark, torch.full_like(mark, 4.0))
+    finally:
+        p.close()
