@@ -1631,6 +1631,8 @@ int run_small(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
     if (!ph.ev_kernel && (rc = cache.get_event(p->device, &ph.ev_kernel)) != SR_OK) return rc;
     if (!ph.d_mem && (rc = cache.get(false, p->device, half, &ph.d_mem, &ph.d_cap)) != SR_OK) return rc;
     SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_kernel, 0));   // the last reader of the device's tables
+    // the first launch, on whichever stream: the event stands for both readers from here on
+    SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_slot[slot], 0));
     const uint32_t vectors = uint32_t(half / 16);
     hipLaunchKernelGGL(sr_table_copy_kernel, dim3((vectors + kSetupBlock - 1) / kSetupBlock), dim3(kSetupBlock), 0,
                        stream, table, static_cast<unsigned char*>(ph.d_mem), vectors);
