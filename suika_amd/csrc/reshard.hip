@@ -67,13 +67,11 @@
 //     Llama2-7B share has 1.44 M tiles per phase; building them on the host
 //     took 0.12 s and a 35 MB upload per phase.
 //   * Tile records and items hold absolute addresses.  When the caller's
-//     pointers change, only the pointer table is rewritten and the emit kernel
+//     pointers change, only the pointer table is uploaded and the emit kernel
 //     writes both again from the descriptors and the device-side buffer
-//     offsets.
-//   * The emit kernel reads descriptors and pointers where the host wrote
-//     them, in pinned memory.  It reads each once; a copy command ahead of it
-//     cost 6 us per change of pointers (GPT-125M block, TP4 -> TP2 into fresh
-//     tensors: 37 us a call with it, 31 without).
+//     offsets.  (Read in place in pinned memory, without the upload, the emit
+//     is 1 us a launch slower: 4096 tiles 33.1 -> 34.1 us.)
+//   * Phases of few tiles have their tables written by the host (run_small).
 
 #include <hip/hip_runtime.h>
 
@@ -779,9 +777,9 @@ constexpr uint64_t kInlineSetupTiles = 65536;
 // Phases of at most this many tiles have their tables written by the host
 // and read from its memory at the first launch on new pointers, which saves
 // the emit kernel.  Above, the tiles' reads over the host link and the host's
-// writes cost more.  A call with new pointers, us, emit / host tables (f32
-// rows of 8 KiB split off): 8 tiles 19.2 / 8.0, 512 20.8 / 9.6, 1024 21.9 /
-// 13.0, 2048 26.7 / 21.3, 4096 37.1 / 38.7.  Launches that repeat the pointers
+// writes cost more.  A call with new pointers, us, upload and emit / host
+// tables (f32 rows of 8 KiB split off): 8 tiles 17.4 / 7.7, 512 17.8 / 9.2,
+// 1024 18.8 / 12.9, 2048 24.8 / 21.2, 4096 36.0 / 38.7.  Launches that repeat the pointers
 // read device memory, as 2048 tiles take 21.4 from the host's and 14.4 from
 // the device's.
 constexpr uint64_t kHostTableTiles = 2048;
@@ -1009,22 +1007,23 @@ struct Phase {
   uint64_t bytes_read = 0;
   uint64_t bytes_written = 0;
   // device state, created on first use: one device allocation carved into
-  // the tables, one pinned host buffer with what the emit kernel reads
+  // the tables, one pinned host buffer for their uploads
   bool ready = false;
   void* d_mem = nullptr;
   size_t d_cap = 0;                     // bytes of d_mem / h_staging as allocated
   size_t h_cap = 0;
+  DevRel* d_rel = nullptr;              // uploaded: descriptors, tile prefix, pointer table
+  uint64_t* d_tile_base = nullptr;
+  uint64_t* d_ptrs = nullptr;
+  EmitChunk* d_chunks = nullptr;
   DevItem* d_items = nullptr;           // built on the device
   DevTile* d_tiles = nullptr;
-  unsigned char* h_staging = nullptr;   // pinned, holds the four tables below
-  DevRel* h_rel = nullptr;
-  uint64_t* h_tile_base = nullptr;
-  EmitChunk* h_chunks = nullptr;
-  uint64_t* h_ptrs = nullptr;           // the pointer table
+  unsigned char* h_staging = nullptr;   // pinned: the uploaded part, in the same layout
+  uint64_t* h_ptrs = nullptr;           // the pointer-table part of h_staging
   std::vector<uint64_t> bound;          // pointer table of the last bind
   bool bound_valid = false;
   hipEvent_t ev_setup = nullptr;        // tile table, offsets and the first bind written
-  hipEvent_t ev_staging = nullptr;      // a later bind done (its reads of h_staging too)
+  hipEvent_t ev_staging = nullptr;      // a later bind done (its copy out of h_staging too)
   hipEvent_t ev_kernel = nullptr;       // last kernel reading d_items
   hipEvent_t ev_bound = nullptr;        // the latest bind: ev_setup or ev_staging (not owned)
   // small phases (kHostTableTiles): two pinned tables in h_staging, written in turn
@@ -1455,19 +1454,19 @@ int setup_offsets(sr_plan* p, hipStream_t stream) {
 }
 
 // The tile and item tables of a phase, from its descriptors and the pointer
-// table, which the kernel reads in pinned host memory.
+// table, all on the device.
 int emit_tables(sr_plan* p, Phase& ph, hipStream_t stream) {
   const uint32_t n_chunks = uint32_t(ph.emit_chunks.size());
   hipLaunchKernelGGL(sr_tile_emit_kernel, dim3(std::min<uint32_t>(n_chunks, 65535u)), dim3(kSetupBlock), 0, stream,
-                     ph.h_rel, ph.h_tile_base, ph.h_chunks, n_chunks, log2u(p->opt.tile_bytes), ph.d_tiles, ph.h_ptrs,
+                     ph.d_rel, ph.d_tile_base, ph.d_chunks, n_chunks, log2u(p->opt.tile_bytes), ph.d_tiles, ph.d_ptrs,
                      p->d_offset, ph.d_items);
   SR_HIP_TRY(hipGetLastError());
   return SR_OK;
 }
 
 // First use of a phase: its descriptors, tile prefix and pointer table go
-// to pinned memory, and one kernel builds the tile table from there and
-// binds the items to `ptrs`, stream-ordered on `stream`.  With
+// up in one copy from pinned memory, then one kernel builds the tile table
+// and binds the items to `ptrs`, stream-ordered on `stream`.  With
 // `mark`, ev_setup marks completion (for a copy kernel on another stream);
 // else the phase's next copy kernel follows on `stream` and its ev_kernel
 // stands for the bind.
@@ -1481,30 +1480,32 @@ int setup_phase(sr_plan* p, Phase& ph, bool needs_offsets, const std::vector<uin
   const uint32_t n = uint32_t(ph.rel.size());
   if (n > 0) {
     const size_t nptr = std::max<size_t>(1, size_t(ph.n_src_base) + ph.n_dst_base);
-    size_t h_end = 0;   // pinned, read by the emit kernel
-    const size_t o_rel = carve(h_end, n * sizeof(DevRel));
-    const size_t o_base = carve(h_end, (size_t(n) + 1) * sizeof(uint64_t));
-    const size_t o_chunk = carve(h_end, ph.emit_chunks.size() * sizeof(EmitChunk));
-    const size_t o_ptr = carve(h_end, nptr * sizeof(uint64_t));
-    size_t d_end = 0;
-    const size_t o_items = carve(d_end, n * sizeof(DevItem));
-    const size_t o_tiles = carve(d_end, ph.n_recs * sizeof(DevTile));
+    size_t end = 0;   // the first three are uploaded (pinned staging, same layout)
+    const size_t o_rel = carve(end, n * sizeof(DevRel));
+    const size_t o_base = carve(end, (size_t(n) + 1) * sizeof(uint64_t));
+    const size_t o_chunk = carve(end, ph.emit_chunks.size() * sizeof(EmitChunk));
+    const size_t o_ptr = carve(end, nptr * sizeof(uint64_t));
+    const size_t up_end = o_ptr + nptr * sizeof(uint64_t);
+    const size_t o_items = carve(end, n * sizeof(DevItem));
+    const size_t o_tiles = carve(end, ph.n_recs * sizeof(DevTile));
     // allocations survive a failed attempt and are reused by the retry
-    if (!ph.d_mem && (rc = cache.get(false, p->device, d_end, &ph.d_mem, &ph.d_cap)) != SR_OK) return rc;
+    if (!ph.d_mem && (rc = cache.get(false, p->device, end, &ph.d_mem, &ph.d_cap)) != SR_OK) return rc;
     if (!ph.h_staging &&
-        (rc = cache.get(true, p->device, h_end, reinterpret_cast<void**>(&ph.h_staging), &ph.h_cap)) != SR_OK)
+        (rc = cache.get(true, p->device, up_end, reinterpret_cast<void**>(&ph.h_staging), &ph.h_cap)) != SR_OK)
       return rc;
     unsigned char* d = static_cast<unsigned char*>(ph.d_mem);
+    ph.d_rel = reinterpret_cast<DevRel*>(d + o_rel);
+    ph.d_tile_base = reinterpret_cast<uint64_t*>(d + o_base);
+    ph.d_ptrs = reinterpret_cast<uint64_t*>(d + o_ptr);
+    ph.d_chunks = reinterpret_cast<EmitChunk*>(d + o_chunk);
     ph.d_items = reinterpret_cast<DevItem*>(d + o_items);
     ph.d_tiles = reinterpret_cast<DevTile*>(d + o_tiles);
-    ph.h_rel = reinterpret_cast<DevRel*>(ph.h_staging + o_rel);
-    ph.h_tile_base = reinterpret_cast<uint64_t*>(ph.h_staging + o_base);
-    ph.h_chunks = reinterpret_cast<EmitChunk*>(ph.h_staging + o_chunk);
     ph.h_ptrs = reinterpret_cast<uint64_t*>(ph.h_staging + o_ptr);
-    std::memcpy(ph.h_rel, ph.rel.data(), n * sizeof(DevRel));
-    std::memcpy(ph.h_tile_base, ph.tile_base.data(), (size_t(n) + 1) * sizeof(uint64_t));
-    std::memcpy(ph.h_chunks, ph.emit_chunks.data(), ph.emit_chunks.size() * sizeof(EmitChunk));
+    std::memcpy(ph.h_staging + o_rel, ph.rel.data(), n * sizeof(DevRel));
+    std::memcpy(ph.h_staging + o_base, ph.tile_base.data(), (size_t(n) + 1) * sizeof(uint64_t));
+    std::memcpy(ph.h_staging + o_chunk, ph.emit_chunks.data(), ph.emit_chunks.size() * sizeof(EmitChunk));
     std::memcpy(ph.h_ptrs, ptrs.data(), ptrs.size() * sizeof(uint64_t));
+    SR_HIP_TRY(hipMemcpyAsync(ph.d_mem, ph.h_staging, up_end, hipMemcpyHostToDevice, stream));
     if (needs_offsets) {
       rc = setup_offsets(p, stream);
       if (rc != SR_OK) return rc;
@@ -1687,15 +1688,17 @@ int run_phase(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
     if (rc != SR_OK) return rc;
     if (setup != stream) SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_setup, 0));
   } else if (rebind) {
-    // Later rebinds run on `stream`, after the latest bind (whose reads of
-    // the staging buffer must be done before the host rewrites it) and after
-    // the phase's previous launch (which may still read the item and tile
-    // tables).
+    // Later rebinds run on `stream`, after the latest bind (whose copy out
+    // of the staging buffer must be done before the host rewrites it) and
+    // after the phase's previous launch (which may still read the item and
+    // pointer tables).
     if (!ph.ev_staging && (rc = table_cache().get_event(p->device, &ph.ev_staging)) != SR_OK) return rc;
     SR_HIP_TRY(hipEventSynchronize(ph.ev_bound));
     std::memcpy(ph.h_ptrs, ptrs.data(), ptrs.size() * sizeof(uint64_t));
     SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_bound, 0));
     SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_kernel, 0));
+    SR_HIP_TRY(hipMemcpyAsync(ph.d_ptrs, ph.h_ptrs, ptrs.size() * sizeof(uint64_t), hipMemcpyHostToDevice,
+                              stream));
     if ((rc = emit_tables(p, ph, stream)) != SR_OK) return rc;
     SR_HIP_TRY(hipEventRecord(ph.ev_staging, stream));
     ph.ev_bound = ph.ev_staging;
