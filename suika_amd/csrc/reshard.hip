@@ -1026,10 +1026,17 @@ struct Phase {
   hipEvent_t ev_staging = nullptr;      // a later bind done (its copy out of h_staging too)
   hipEvent_t ev_kernel = nullptr;       // last kernel reading d_items
   hipEvent_t ev_bound = nullptr;        // the latest bind: ev_setup or ev_staging (not owned)
-  // small phases (kHostTableTiles): two pinned tables in h_staging, written in turn
+  // small phases (kHostTableTiles): two pinned tables, written in turn, and a
+  // device copy of the latest.  Memory of their own: a first use on a
+  // capturing stream takes the blocks above, of other sizes, and may fail
+  // after it did.
+  unsigned char* h_tables = nullptr;
+  unsigned char* d_tables = nullptr;
+  size_t h_tables_cap = 0;
+  size_t d_tables_cap = 0;
   int slot = 0;
   hipEvent_t ev_slot[2] = {};           // last kernel reading the table
-  bool on_device = false;               // the tables are in d_mem too
+  bool on_device = false;               // the tables are in d_tables too
 };
 
 }  // namespace
@@ -1602,11 +1609,11 @@ int run_small(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
   const size_t o_tiles = carve(end, ph.n_recs * sizeof(DevTile));
   const size_t half = carve(end, 0);
   int rc;
-  if (!ph.h_staging &&
-      (rc = cache.get(true, p->device, 2 * half, reinterpret_cast<void**>(&ph.h_staging), &ph.h_cap)) != SR_OK)
+  if (!ph.h_tables &&
+      (rc = cache.get(true, p->device, 2 * half, reinterpret_cast<void**>(&ph.h_tables), &ph.h_tables_cap)) != SR_OK)
     return rc;
   const int slot = rebind ? ph.slot ^ 1 : ph.slot;
-  unsigned char* table = ph.h_staging + slot * half;
+  unsigned char* table = ph.h_tables + slot * half;
   if (rebind) {
     if (ph.ev_slot[slot]) SR_HIP_TRY(hipEventSynchronize(ph.ev_slot[slot]));
     else if ((rc = cache.get_event(p->device, &ph.ev_slot[slot])) != SR_OK) return rc;
@@ -1630,13 +1637,15 @@ int run_small(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
   if (!rebind && !ph.on_device) {
     if (!ph.ev_setup && (rc = cache.get_event(p->device, &ph.ev_setup)) != SR_OK) return rc;
     if (!ph.ev_kernel && (rc = cache.get_event(p->device, &ph.ev_kernel)) != SR_OK) return rc;
-    if (!ph.d_mem && (rc = cache.get(false, p->device, half, &ph.d_mem, &ph.d_cap)) != SR_OK) return rc;
+    if (!ph.d_tables &&
+        (rc = cache.get(false, p->device, half, reinterpret_cast<void**>(&ph.d_tables), &ph.d_tables_cap)) != SR_OK)
+      return rc;
     SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_kernel, 0));   // the last reader of the device's tables
     // the first launch, on whichever stream: the event stands for both readers from here on
     SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_slot[slot], 0));
     const uint32_t vectors = uint32_t(half / 16);
     hipLaunchKernelGGL(sr_table_copy_kernel, dim3((vectors + kSetupBlock - 1) / kSetupBlock), dim3(kSetupBlock), 0,
-                       stream, table, static_cast<unsigned char*>(ph.d_mem), vectors);
+                       stream, table, ph.d_tables, vectors);
     SR_HIP_TRY(hipGetLastError());
     SR_HIP_TRY(hipEventRecord(ph.ev_setup, stream));
     SR_HIP_TRY(hipEventRecord(ph.ev_slot[slot], stream));
@@ -1644,7 +1653,7 @@ int run_small(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
   } else if (ph.on_device) {
     SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_setup, 0));
   }
-  if (ph.on_device) table = static_cast<unsigned char*>(ph.d_mem);
+  if (ph.on_device) table = ph.d_tables;
   rc = launch_copy(p->opt, ph, kind, reinterpret_cast<DevItem*>(table + o_items),
                    reinterpret_cast<DevTile*>(table + o_tiles), ph.on_device, stream);
   if (rc != SR_OK) return rc;
@@ -1666,7 +1675,7 @@ int run_phase(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
     if (cap == hipStreamCaptureStatusNone) return run_small(p, ph, kind, ptrs, rebind, stream);
     // A graph would replay reads of tables that the host writes again; a
     // phase whose first use is captured keeps the device tables below.
-    if (ph.h_staging) return fail(SR_EHIP, "a plan that has run before cannot be captured into a graph");
+    if (ph.h_tables) return fail(SR_EHIP, "a plan that has run before cannot be captured into a graph");
   }
   if (!ph.ready) {
     // A phase's first use builds its tables and binds the pointers.  They
@@ -1723,6 +1732,8 @@ void free_phase(Phase& ph, int device) {
     if (ev) (void)hipEventSynchronize(ev);
   cache.put(false, device, ph.d_mem, ph.d_cap);
   cache.put(true, device, ph.h_staging, ph.h_cap);
+  cache.put(false, device, ph.d_tables, ph.d_tables_cap);
+  cache.put(true, device, ph.h_tables, ph.h_tables_cap);
   for (hipEvent_t ev : {ph.ev_setup, ph.ev_staging, ph.ev_kernel, ph.ev_slot[0], ph.ev_slot[1]}) cache.put_event(device, ev);
   ph = Phase();
 }
