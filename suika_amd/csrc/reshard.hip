@@ -1024,8 +1024,9 @@ struct Phase {
   bool bound_valid = false;
   hipEvent_t ev_setup = nullptr;        // tile table, offsets and the first bind written
   hipEvent_t ev_staging = nullptr;      // a later bind done (its copy out of h_staging too)
-  hipEvent_t ev_kernel = nullptr;       // last kernel reading d_items
-  hipEvent_t ev_bound = nullptr;        // the latest bind: ev_setup or ev_staging (not owned)
+  hipEvent_t ev_kernel = nullptr;       // last copy kernel reading the device's tables, and all before it
+  hipEvent_t ev_bound = nullptr;        // the latest bind: ev_setup, ev_staging or ev_kernel (not owned)
+  hipEvent_t ev_tail = nullptr;         // the latest bind or copy kernel (not owned)
   // small phases (kHostTableTiles): two pinned tables, written in turn, and a
   // device copy of the latest.  Memory of their own: a first use on a
   // capturing stream takes the blocks above, of other sizes, and may fail
@@ -1522,9 +1523,9 @@ int setup_phase(sr_plan* p, Phase& ph, bool needs_offsets, const std::vector<uin
   }
   if (mark) {
     SR_HIP_TRY(hipEventRecord(ph.ev_setup, stream));
-    ph.ev_bound = ph.ev_setup;
+    ph.ev_bound = ph.ev_tail = ph.ev_setup;
   } else {
-    ph.ev_bound = ph.ev_kernel;   // recorded after the copy kernel, which follows on `stream`
+    ph.ev_bound = ph.ev_tail = ph.ev_kernel;   // recorded after the copy kernel, which follows on `stream`
   }
   ph.bound = ptrs;
   ph.bound_valid = true;
@@ -1634,30 +1635,30 @@ int run_small(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
     ph.bound = ptrs;
     ph.bound_valid = true;
   }
-  if (!rebind && !ph.on_device) {
-    if (!ph.ev_setup && (rc = cache.get_event(p->device, &ph.ev_setup)) != SR_OK) return rc;
+  if (!rebind) {
+    // Each launch that reads the device's tables follows the one before it,
+    // whichever streams they are on: the event stands for all of them.
     if (!ph.ev_kernel && (rc = cache.get_event(p->device, &ph.ev_kernel)) != SR_OK) return rc;
-    if (!ph.d_tables &&
-        (rc = cache.get(false, p->device, half, reinterpret_cast<void**>(&ph.d_tables), &ph.d_tables_cap)) != SR_OK)
-      return rc;
-    SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_kernel, 0));   // the last reader of the device's tables
-    // the first launch, on whichever stream: the event stands for both readers from here on
-    SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_slot[slot], 0));
-    const uint32_t vectors = uint32_t(half / 16);
-    hipLaunchKernelGGL(sr_table_copy_kernel, dim3((vectors + kSetupBlock - 1) / kSetupBlock), dim3(kSetupBlock), 0,
-                       stream, table, ph.d_tables, vectors);
-    SR_HIP_TRY(hipGetLastError());
-    SR_HIP_TRY(hipEventRecord(ph.ev_setup, stream));
-    SR_HIP_TRY(hipEventRecord(ph.ev_slot[slot], stream));
-    ph.on_device = true;
-  } else if (ph.on_device) {
-    SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_setup, 0));
+    SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_kernel, 0));
+    if (!ph.on_device) {
+      if (!ph.d_tables &&
+          (rc = cache.get(false, p->device, half, reinterpret_cast<void**>(&ph.d_tables), &ph.d_tables_cap)) != SR_OK)
+        return rc;
+      // the first launch, on whichever stream: the event stands for both readers from here on
+      SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_slot[slot], 0));
+      const uint32_t vectors = uint32_t(half / 16);
+      hipLaunchKernelGGL(sr_table_copy_kernel, dim3((vectors + kSetupBlock - 1) / kSetupBlock), dim3(kSetupBlock), 0,
+                         stream, table, ph.d_tables, vectors);
+      SR_HIP_TRY(hipGetLastError());
+      SR_HIP_TRY(hipEventRecord(ph.ev_slot[slot], stream));
+    }
+    table = ph.d_tables;
   }
-  if (ph.on_device) table = ph.d_tables;
   rc = launch_copy(p->opt, ph, kind, reinterpret_cast<DevItem*>(table + o_items),
-                   reinterpret_cast<DevTile*>(table + o_tiles), ph.on_device, stream);
+                   reinterpret_cast<DevTile*>(table + o_tiles), !rebind, stream);
   if (rc != SR_OK) return rc;
-  SR_HIP_TRY(hipEventRecord(ph.on_device ? ph.ev_kernel : ph.ev_slot[slot], stream));
+  SR_HIP_TRY(hipEventRecord(rebind ? ph.ev_slot[slot] : ph.ev_kernel, stream));
+  ph.on_device = !rebind;
   return SR_OK;
 }
 
@@ -1710,16 +1711,18 @@ int run_phase(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
                               stream));
     if ((rc = emit_tables(p, ph, stream)) != SR_OK) return rc;
     SR_HIP_TRY(hipEventRecord(ph.ev_staging, stream));
-    ph.ev_bound = ph.ev_staging;
+    ph.ev_bound = ph.ev_tail = ph.ev_staging;
     ph.bound = ptrs;
     ph.bound_valid = true;
   } else {
-    // the latest bind (which follows the tables on its stream)
-    SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_bound, 0));
+    // the launch before, on whichever stream: the next bind, or the plan's
+    // end, waits for the latest launch alone
+    SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_tail, 0));
   }
 
   if ((rc = launch_copy(p->opt, ph, kind, ph.d_items, ph.d_tiles, true, stream)) != SR_OK) return rc;
   SR_HIP_TRY(hipEventRecord(ph.ev_kernel, stream));
+  ph.ev_tail = ph.ev_kernel;
   return SR_OK;
 }
 

@@ -442,12 +442,39 @@ void capture_fails() {
   }
 }
 
+// Launches of one binding on two streams, then other bindings, all while the
+// first stream's work is held back; at last the plan goes, and its memory to
+// another plan.
+void two_streams(uint64_t tiles, int first, int repeats) {
+  Job j(tiles, 3);
+  ok(j.gather(2, 1), "gather");   // a binding before, so that this one is not the plan's first
+  for (int i = 0; i < first; ++i) ok(j.gather(0, 1), "gather");
+  for (int i = 0; i < repeats; ++i) ok(j.gather(0, 2), "gather");
+  for (int k : {1, 2, 1})
+    for (int i = 0; i < 2; ++i) ok(j.gather(k, 2), "gather");
+  drain({2, 1});
+  for (int k = 0; k < 3; ++k) j.check(k, "two streams");
+
+  Job a(tiles, 2);
+  ok(a.gather(1, 1), "gather");
+  for (int i = 0; i < first; ++i) ok(a.gather(0, 1), "gather");
+  ok(a.gather(0, 2), "gather");
+  a.close();
+  Job b(tiles, 1, 25, 9);
+  for (int i = 0; i < 2; ++i) ok(b.gather(0, 3), "gather");
+  drain({3, 2, 1});
+  a.check(0, "destroyed while a stream still runs");
+  b.check(0, "memory of a destroyed plan");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "routes") routes();
   else if (what == "capture_fails") capture_fails();
+  else if (what == "two_streams_small") for (int first : {1, 2, 3}) for (int n : {0, 1, 2}) two_streams(kSmall, first, n);
+  else if (what == "two_streams_large") for (int first : {1, 2, 3}) for (int n : {0, 1, 2}) two_streams(kLarge, first, n);
   else die("no such scenario");
   check_guards("end");
   std::puts("ok");

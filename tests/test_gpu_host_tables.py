@@ -1,7 +1,8 @@
 """Small phases: tables written by the host at the first launch on new
 pointers, device tables from the second.  Around the tile count where the
 other route begins, both give torch's bytes, also where bindings take turns
-without a host synchronisation.  All exact."""
+without a host synchronisation, and where launches of one binding are on two
+streams.  All exact."""
 import ctypes
 
 import pytest
@@ -100,6 +101,51 @@ def test_bindings_in_turn(tiles, cols, split):
             p.check(srcs[i], dsts[i])
     finally:
         p.close()
+
+
+@pytest.mark.parametrize("tiles", [64, LIMIT, LIMIT + 1])
+@pytest.mark.parametrize("first", [1, 2, 3])
+def test_two_streams(tiles, first):
+    """Launches of one binding on a stream that is held up by other work and
+    then on a free one, where other bindings follow, with no host wait; then a
+    plan destroyed while its first stream still runs, and its table memory in
+    another plan's hands."""
+    print(f"[gpu host tables] two streams, {tiles} tiles, {first} launches on the first", flush=True)
+    p, a, b = Plan(tiles), Plan(tiles), Plan(tiles)
+    srcs, dsts = [p.src(i) for i in range(3)], [p.dst() for _ in range(3)]
+    last_src, last_dst = [p.src(i) for i in (3, 4)], [p.dst() for _ in range(2)]
+    held = torch.randn(1 << 28, device="cuda")
+    copy = torch.empty_like(held)
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    try:
+        with torch.cuda.stream(s1):
+            p.gather(srcs[2], dsts[2])
+            for _ in range(8):
+                copy.copy_(held)
+            for _ in range(first):
+                p.gather(srcs[0], dsts[0])
+        with torch.cuda.stream(s2):
+            p.gather(srcs[0], dsts[0])
+            for i in (1, 1, 2, 2, 1):
+                p.gather(srcs[i], dsts[i])
+        with torch.cuda.stream(s1):
+            for _ in range(8):
+                copy.copy_(held)
+            for _ in range(first):
+                a.gather(last_src[0], last_dst[0])
+        with torch.cuda.stream(s2):
+            a.gather(last_src[0], last_dst[0])
+        a.L.sr_plan_destroy(a.h)
+        with torch.cuda.stream(s2):
+            for _ in range(2):
+                b.gather(last_src[1], last_dst[1])
+        torch.cuda.synchronize()
+        for s, d in zip(srcs + last_src, dsts + last_dst):
+            p.check(s, d)
+    finally:
+        p.close()
+        b.close()
 
 
 def test_graph_capture_stays_refused():

@@ -24,7 +24,7 @@ def model(tmp_path_factory):
     return out / "model"
 
 
-@pytest.mark.parametrize("scenario", ["routes", "capture_fails"])
+@pytest.mark.parametrize("scenario", ["routes", "capture_fails", "two_streams_small", "two_streams_large"])
 def test_scenario(model, scenario):
     res = subprocess.run([str(model), scenario], capture_output=True, text=True, timeout=300)
     assert res.returncode == 0 and res.stdout.endswith("ok\n"), res.stdout + res.stderr
