@@ -19,6 +19,7 @@
 //   * Items are cut into tiles of `tile_bytes` (16 KiB) source bytes; one
 //     workgroup (1024 lanes = 16 wave64) moves one tile, 16 bytes per lane,
 //     and the grid is the tile count (or a grid-stride loop when capped).
+//     Phases of few, small or several-pass tiles have other workgroups (Shape).
 //     Tiles balance the work whatever the tensor sizes (8 KB norms to GB
 //     embeddings).
 //   * A lane loads once, stores once and ends.  Two workgroups fill a compute
@@ -122,20 +123,18 @@ int dtype_size(int32_t dt) {
 
 namespace {
 
-// A copy workgroup: 1024 lanes that each hold one 16-byte vector (or as many
-// narrower ones as make 16 bytes) of a 16 KiB tile.
-constexpr int kBlock = 1024;
-constexpr uint32_t kPassBytes = kBlock * 16;
+// What the largest copy workgroup, 1024 lanes, moves with one 16-byte vector
+// (or as many narrower ones as make 16 bytes) per lane: a tile.
+constexpr uint32_t kPassBytes = 16384;
 constexpr uint32_t kDefaultTileBytes = kPassBytes;
 constexpr uint64_t kBufAlign = 256;
 // Segments of the tile list, one per accelerator complex die (XCD) of an
 // MI355X; the dies take workgroups round-robin.
 constexpr uint32_t kXcds = 8;
-constexpr uint32_t kMaxGrid = 0xffffffffu / kBlock;    // grid work-items stay below 2^32
 // A RECAST item that writes the f32 copy and the bf16 copy moves 2.5x its
 // source bytes (a COPY item 2x); its tiles, as plans count them, hold
-// tile_bytes >> this many source bytes.  A workgroup takes two of them: it
-// has lanes for tile_bytes.
+// tile_bytes >> this many source bytes.  A workgroup takes two of them where
+// it has lanes for both (record_bytes).
 constexpr uint32_t kRecastTileShift = 1;
 
 // ---------------------------------------------------------------- errors
@@ -432,8 +431,9 @@ constexpr uint32_t kAheadStep = 4;
 struct Ahead {
   const DevTile* tiles;
   uint32_t i, n, lane;
+  template <int B>
   __device__ __forceinline__ void touch() const {
-    if (lane >= kBlock - 64 && i % kAheadStep == 0 && i + kAhead < n) {
+    if (lane >= B - 64 && i % kAheadStep == 0 && i + kAhead < n) {
       const uint32_t x = __hip_atomic_load(&tiles[i + kAhead].info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       asm volatile("" ::"v"(x));
     }
@@ -443,35 +443,44 @@ struct Ahead {
 // A tile of at least 16 contiguous bytes, at any alignment: 16 bytes per
 // lane, the last vector moved back to end with the tile (it then writes
 // bytes of its neighbour again, with the same values).
-template <uint32_t KIND, bool NT, Policy POLICY>
+template <uint32_t KIND, bool NT, Policy POLICY, int B, int U>
 __device__ __forceinline__ void contiguous_tile(const Regions& r, uint32_t nbytes, const Ahead& ahead) {
-  for (uint32_t base = 0; base < nbytes; base += kPassBytes) {
-    const uint32_t off = contiguous_vec(base + ahead.lane * 16, nbytes);
-    VecOf<16>::type v(0);
-    if constexpr (KIND != kKindZero) {
-      v = ld<16, NT>(r.src, off);
-      if (base == 0) ahead.touch();
+  for (uint32_t base = 0; base < nbytes; base += B * U * 16) {
+    uint32_t off[U];
+    VecOf<16>::type v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      off[u] = contiguous_vec(base + (u * B + ahead.lane) * 16, nbytes);
+      v[u] = VecOf<16>::type(0);
+      if constexpr (KIND != kKindZero) v[u] = ld<16, NT>(r.src, off[u]);
     }
-    put<KIND, 16, POLICY>(r, Place{off, off, off >> 1}, v);
+    if (KIND != kKindZero && base == 0) ahead.touch<B>();
+#pragma unroll
+    for (int u = 0; u < U; ++u) put<KIND, 16, POLICY>(r, Place{off[u], off[u], off[u] >> 1}, v[u]);
   }
 }
 
 // A tile of rows of a multiple of 16 bytes, at any alignment: 16 bytes per lane.
-template <uint32_t KIND, bool NT, Policy POLICY>
+template <uint32_t KIND, bool NT, Policy POLICY, int B, int U>
 __device__ __forceinline__ void rows_tile(const Regions& r, const DevItem& it, uint32_t column, uint32_t nbytes,
                                           const Ahead& ahead) {
   const RowMap rows = row_map(it, column);
   const uint32_t ss = uint32_t(it.src_stride), ds = uint32_t(it.dst_stride), hs = uint32_t(it.dst2_stride);
-  for (uint32_t base = 0; base < nbytes; base += kPassBytes) {
-    const uint32_t b = base + ahead.lane * 16;
-    uint32_t row, col;
-    rows.at(b, row, col);
-    const bool in = b < nbytes;
-    const Place at = {in ? row * ss + col : kNowhere, in ? row * ds + col : kNowhere,
-                      in ? row * hs + (col >> 1) : kNowhere};
-    const VecOf<16>::type v = ld<16, NT>(r.src, at.src);
-    if (base == 0) ahead.touch();
-    put<KIND, 16, POLICY>(r, at, v);
+  for (uint32_t base = 0; base < nbytes; base += B * U * 16) {
+    Place at[U];
+    VecOf<16>::type v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t b = base + (u * B + ahead.lane) * 16;
+      uint32_t row, col;
+      rows.at(b, row, col);
+      const bool in = b < nbytes;
+      at[u] = {in ? row * ss + col : kNowhere, in ? row * ds + col : kNowhere, in ? row * hs + (col >> 1) : kNowhere};
+      v[u] = ld<16, NT>(r.src, at[u].src);
+    }
+    if (base == 0) ahead.touch<B>();
+#pragma unroll
+    for (int u = 0; u < U; ++u) put<KIND, 16, POLICY>(r, at[u], v[u]);
   }
 }
 
@@ -496,7 +505,7 @@ __device__ __forceinline__ Regions row_regions(const DevItem& it, uint64_t row) 
 // that runs over the end of its row (rows that are no multiple of 16 bytes;
 // not RECAST) becomes two, the last 16 bytes of that row and the first 16 of
 // the next; the bytes that neighbouring lanes write too have the same values.
-template <bool NT>
+template <bool NT, int B>
 __device__ __forceinline__ void wide_tile(const DevItem& it, const DevTile& t, uint32_t nbytes, const Ahead& ahead) {
   const bool strided = it.row_bytes != 0, recast = (it.flags & 0xfu) == kKindRecast;
   const Regions r = strided ? row_regions(it, t.src)
@@ -504,7 +513,7 @@ __device__ __forceinline__ void wide_tile(const DevItem& it, const DevTile& t, u
                                       region(it.dst2 + ((t.src - it.src) >> 1), it.dst2 ? nbytes >> 1 : 0)};
   const RowMap rows = row_map(it, uint32_t(t.dst));
   const uint32_t ss = uint32_t(it.src_stride), ds = uint32_t(it.dst_stride), hs = uint32_t(it.dst2_stride);
-  for (uint32_t base = 0; base < nbytes; base += kPassBytes) {
+  for (uint32_t base = 0; base < nbytes; base += B * 16) {
     const uint32_t b = base + ahead.lane * 16;
     Place at, at2{kNowhere, kNowhere, kNowhere};
     if (strided) {
@@ -518,7 +527,7 @@ __device__ __forceinline__ void wide_tile(const DevItem& it, const DevTile& t, u
     }
     const VecOf<16>::type v = ld<16, NT>(r.src, at.src), w = ld<16, NT>(r.src, at2.src);
     const VecOf<8>::type h = to_bf16<4>(v);
-    if (base == 0) ahead.touch();
+    if (base == 0) ahead.touch<B>();
 #define SR_PUT(POLICY)                                \
   do {                                                \
     st<16, POLICY>(r.dst, at.dst, v);                 \
@@ -535,13 +544,13 @@ __device__ __forceinline__ void wide_tile(const DevItem& it, const DevTile& t, u
 // width apart: each vector's lines are then written by one wave (side by
 // side f32 rows of 16396 bytes: 5.7 TB/s, with the vectors of a lane a
 // workgroup's width apart 5.2).
-template <uint32_t KIND, int VB, bool NT, Policy POLICY>
+template <uint32_t KIND, int VB, bool NT, Policy POLICY, int B>
 __device__ __forceinline__ void narrow_vectors(const Regions& r, const DevItem& it, uint32_t column, uint32_t nbytes,
                                                const Ahead& ahead) {
   constexpr int U = VB == 8 ? 2 : 4;
   constexpr uint32_t kStep = 64 * VB;
   const RowMap rows = row_map(it, column);
-  for (uint32_t base = 0; base < nbytes; base += kBlock * VB * U) {
+  for (uint32_t base = 0; base < nbytes; base += B * VB * U) {
     uint32_t b = base + (ahead.lane >> 6) * (U * kStep) + (ahead.lane & 63) * VB;
     RowWalk walk(rows, b, kStep, uint32_t(it.src_stride), uint32_t(it.dst_stride), uint32_t(it.dst2_stride));
     Place at[U];
@@ -554,40 +563,41 @@ __device__ __forceinline__ void narrow_vectors(const Regions& r, const DevItem& 
       b += kStep;
       walk.advance();
     }
-    if (base == 0) ahead.touch();
+    if (base == 0) ahead.touch<B>();
 #pragma unroll
     for (int u = 0; u < U; ++u) put<KIND, VB, POLICY>(r, at[u], v[u]);
   }
 }
 
-template <bool NT>
+template <bool NT, int B>
 __device__ __forceinline__ void narrow_tile(const DevItem& it, const DevTile& t, uint32_t nbytes, const Ahead& ahead) {
   const bool strided = it.row_bytes != 0, merge = !NT || (it.flags & kItemMerge);
   const uint32_t lv = (it.flags >> 4) & 0xfu, column = strided ? uint32_t(t.dst) : 0;
   const Regions r = row_regions(it, strided ? t.src : 0);
   constexpr Policy kPart = NT ? kStream : kCached;
   if ((it.flags & 0xfu) == kKindRecast) {
-    if (merge) narrow_vectors<kKindRecast, 4, NT, kCached>(r, it, column, nbytes, ahead);
-    else narrow_vectors<kKindRecast, 4, NT, kPart>(r, it, column, nbytes, ahead);
+    if (merge) narrow_vectors<kKindRecast, 4, NT, kCached, B>(r, it, column, nbytes, ahead);
+    else narrow_vectors<kKindRecast, 4, NT, kPart, B>(r, it, column, nbytes, ahead);
   } else if (lv == 3) {   // streamed: kOpRows8, kOpRows4, or one small piece
-    narrow_vectors<kKindCopy, 8, NT, kCached>(r, it, column, nbytes, ahead);
+    narrow_vectors<kKindCopy, 8, NT, kCached, B>(r, it, column, nbytes, ahead);
   } else if (lv == 2) {
-    narrow_vectors<kKindCopy, 4, NT, kCached>(r, it, column, nbytes, ahead);
+    narrow_vectors<kKindCopy, 4, NT, kCached, B>(r, it, column, nbytes, ahead);
   } else if (lv == 1) {
-    if (merge) narrow_vectors<kKindCopy, 2, NT, kCached>(r, it, column, nbytes, ahead);
-    else narrow_vectors<kKindCopy, 2, NT, kPart>(r, it, column, nbytes, ahead);
+    if (merge) narrow_vectors<kKindCopy, 2, NT, kCached, B>(r, it, column, nbytes, ahead);
+    else narrow_vectors<kKindCopy, 2, NT, kPart, B>(r, it, column, nbytes, ahead);
   } else {
-    if (merge) narrow_vectors<kKindCopy, 1, NT, kCached>(r, it, column, nbytes, ahead);
-    else narrow_vectors<kKindCopy, 1, NT, kPart>(r, it, column, nbytes, ahead);
+    if (merge) narrow_vectors<kKindCopy, 1, NT, kCached, B>(r, it, column, nbytes, ahead);
+    else narrow_vectors<kKindCopy, 1, NT, kPart, B>(r, it, column, nbytes, ahead);
   }
 }
 
 // One vector at a time through 64-bit addresses: strided items whose tiles
 // span 2 GiB or more of an object (a few bytes of very long rows).
+template <int B>
 __device__ __forceinline__ void far_tile(const DevItem& it, const DevTile& t, uint32_t nbytes, uint32_t lane) {
   const uint32_t lv = (it.flags >> 4) & 0xfu, kind = it.flags & 0xfu;
   const RowMap rows = row_map(it, uint32_t(t.dst));
-  for (uint32_t b = lane << lv; b < nbytes; b += kBlock << lv) {
+  for (uint32_t b = lane << lv; b < nbytes; b += B << lv) {
     uint32_t row, col;
     rows.at(b, row, col);
     const uint64_t q = t.src + row;
@@ -622,7 +632,7 @@ __device__ __forceinline__ void far_tile(const DevItem& it, const DevTile& t, ui
 // of segment p % kXcds: each die walks one contiguous part of the list, and
 // of the records.  Positions p, p + stride, ... below n_pos are this
 // workgroup's; `stride` is the grid.
-template <bool NT>
+template <bool NT, int B, int U>
 __device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, const DevTile* __restrict__ tiles,
                                            uint32_t n_tiles, uint32_t seg, uint32_t n_pos, uint32_t stride,
                                            uint32_t n_ahead) {
@@ -640,41 +650,42 @@ __device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, co
       constexpr Policy kWhole = NT ? kThrough : kCached, kPartial = NT ? kStream : kCached;
       const Region none = region(0, 0);
       if (__builtin_expect(op == kOpCopy, 1)) {
-        contiguous_tile<kKindCopy, NT, kWhole>(Regions{region(t.src, nbytes), region(t.dst, nbytes), none}, nbytes,
-                                               ahead);
+        contiguous_tile<kKindCopy, NT, kWhole, B, U>(Regions{region(t.src, nbytes), region(t.dst, nbytes), none},
+                                                     nbytes, ahead);
       } else if (__builtin_expect(op == kOpRows, 1)) {
         const DevItem it = items[t.item];
-        rows_tile<kKindCopy, NT, kWhole>(Regions{region(it.src + t.src * it.src_stride, it.src ? kNearBytes : 0),
-                                                 region(it.dst + t.src * it.dst_stride, kNearBytes), none},
-                                         it, uint32_t(t.dst), nbytes, ahead);
+        rows_tile<kKindCopy, NT, kWhole, B, U>(
+            Regions{region(it.src + t.src * it.src_stride, it.src ? kNearBytes : 0),
+                    region(it.dst + t.src * it.dst_stride, kNearBytes), none},
+            it, uint32_t(t.dst), nbytes, ahead);
       } else if (__builtin_expect(op == kOpRecast, 1)) {
         const uint64_t half = items[t.item].dst2 + ((t.src - items[t.item].src) >> 1);
-        contiguous_tile<kKindRecast, NT, kWhole>(
+        contiguous_tile<kKindRecast, NT, kWhole, B, U>(
             Regions{region(t.src, nbytes), region(t.dst, t.dst ? nbytes : 0), region(half, nbytes >> 1)}, nbytes,
             ahead);
       } else if (__builtin_expect(op == kOpZero, 1)) {
-        contiguous_tile<kKindZero, NT, kWhole>(Regions{none, region(t.dst, nbytes), none}, nbytes, ahead);
+        contiguous_tile<kKindZero, NT, kWhole, B, U>(Regions{none, region(t.dst, nbytes), none}, nbytes, ahead);
       } else if (__builtin_expect(op == kOpRecastRows, 1)) {
         const DevItem it = items[t.item];
-        rows_tile<kKindRecast, NT, kWhole>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
+        rows_tile<kKindRecast, NT, kWhole, B, U>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
       } else if (op == kOpShifted) {
-        contiguous_tile<kKindCopy, NT, kPartial>(Regions{region(t.src, nbytes), region(t.dst, nbytes), none}, nbytes,
-                                                 ahead);
+        contiguous_tile<kKindCopy, NT, kPartial, B, U>(Regions{region(t.src, nbytes), region(t.dst, nbytes), none},
+                                                       nbytes, ahead);
       } else if (op == kOpRowsPart) {
         const DevItem it = items[t.item];
-        rows_tile<kKindCopy, NT, kPartial>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
+        rows_tile<kKindCopy, NT, kPartial, B, U>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
       } else if (op == kOpRows8) {
         const DevItem it = items[t.item];
-        narrow_vectors<kKindCopy, 8, NT, kPartial>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
+        narrow_vectors<kKindCopy, 8, NT, kPartial, B>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
       } else if (op == kOpRows4) {
         const DevItem it = items[t.item];
-        narrow_vectors<kKindCopy, 4, NT, kPartial>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
+        narrow_vectors<kKindCopy, 4, NT, kPartial, B>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
       } else if (op == kOpNarrow) {
-        narrow_tile<NT>(items[t.item], t, nbytes, ahead);
+        narrow_tile<NT, B>(items[t.item], t, nbytes, ahead);
       } else if (op == kOpWide) {
-        wide_tile<NT>(items[t.item], t, nbytes, ahead);
+        wide_tile<NT, B>(items[t.item], t, nbytes, ahead);
       } else {
-        far_tile(items[t.item], t, nbytes, lane);
+        far_tile<B>(items[t.item], t, nbytes, lane);
       }
     }
     p += stride;
@@ -682,20 +693,49 @@ __device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, co
 }
 
 // Three entry points with one body, so profiles tell the phases apart.  Eight
-// waves per SIMD (two workgroups per compute unit) need at most 64 vector
+// waves per SIMD (2048 lanes per compute unit) need at most 64 vector
 // registers and, the trap handler's 16 included, 96 scalar ones each: with
-// 84 of its own the kernel ran one workgroup per unit and lost 15%.
-#define SR_COPY_KERNEL(NAME)                                                                                      \
-  template <bool NT>                                                                                              \
-  __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(8))) void NAME(    \
-      const DevItem* __restrict__ items, const DevTile* __restrict__ tiles, uint32_t n_tiles, uint32_t seg,       \
-      uint32_t n_pos, uint32_t stride, uint32_t n_ahead) {                                                        \
-    exec_tiles<NT>(items, tiles, n_tiles, seg, n_pos, stride, n_ahead);                                           \
+// 84 of its own the kernel ran half the waves and lost 15%.
+#define SR_COPY_KERNEL(NAME)                                                                                 \
+  template <bool NT, int B, int U>                                                                           \
+  __global__ __launch_bounds__(B) __attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(8))) void NAME(    \
+      const DevItem* __restrict__ items, const DevTile* __restrict__ tiles, uint32_t n_tiles, uint32_t seg,  \
+      uint32_t n_pos, uint32_t stride, uint32_t n_ahead) {                                                   \
+    exec_tiles<NT, B, U>(items, tiles, n_tiles, seg, n_pos, stride, n_ahead);                                \
   }
 SR_COPY_KERNEL(sr_pack_kernel)
 SR_COPY_KERNEL(sr_unpack_kernel)
 SR_COPY_KERNEL(sr_gather_kernel)
 #undef SR_COPY_KERNEL
+
+// The kernels' workgroups: lanes, and 16-byte vectors that a lane holds at
+// once.  One vector in each of 1024 lanes is the best for the tiles of a large
+// phase; the others are for
+//   * tiles of few vectors, whose workgroups cost more to start than to run:
+//     256 lanes for a mean of 7 KiB or less (us; 1024 / 512 / 256 lanes:
+//     60000 pieces of 1000 bytes 135 / 87 / 46, 4096-byte tiles of 1 GiB
+//     744 / 473 / 325, 8192-byte ones 404 / 329 / 340), 512 lanes for 12 KiB
+//     or less (pieces of 10000 bytes 88 / 76 / 76; of 14000 77 / 75 / 77;
+//     60000 pieces of 1000 bytes among 1 GiB, mean 9 KiB, 425 / 372 / 399);
+//   * few tiles, where each compute unit takes a handful in turn and more of
+//     them side by side hide the way to a tile's first load: 512 lanes of two
+//     vectors up to 5120 tiles (strided, 2624 tiles 18.2 / 15.7 us, 4000
+//     24.5 / 21.7, 6000 36.5 / 36.5);
+//   * grids capped at 512 workgroups or less, the same (1 GiB, 64 workgroups
+//     1123 / 1026 us, 256 421 / 378, 512 394 / 388);
+//   * tiles of more than one pass: two vectors in each of 1024 lanes (64 KiB
+//     tiles, columns merged 381 / 356 us with one / two).
+enum Shape { kWide, kSmall, kTiny, kLong };
+
+constexpr uint32_t shape_lanes(Shape s) { return s == kSmall ? 512 : s == kTiny ? 256 : 1024; }
+
+Shape pick_shape(uint64_t n_recs, uint64_t bytes, uint32_t tile_bytes, uint32_t max_blocks) {
+  const uint64_t mean = bytes / n_recs;
+  if (mean <= 7 * 1024) return kTiny;
+  if (tile_bytes > kPassBytes) return kLong;
+  if (mean <= 12 * 1024 || n_recs <= 5120 || (max_blocks != 0 && max_blocks <= 512)) return kSmall;
+  return kWide;
+}
 
 // ------------------------------------------------- device-side plan binding
 // The host keeps O(pieces) descriptors and the prefix sum of their tile
@@ -712,6 +752,7 @@ enum : uint32_t {
   kRelSrcBuf = 1u << 16,   // source side is a peer buffer at the piece's offset
   kRelDstBuf = 1u << 17,   // destination side is a peer buffer at the piece's offset
   kRelFar = 1u << 18,      // kOpFar
+  kRelShiftBit = 20,       // bits 20-24: log2 of the source bytes of a tile record
 };
 
 struct alignas(8) DevRel {
@@ -725,7 +766,7 @@ struct alignas(8) DevRel {
   uint32_t row_bytes;      // 0 = contiguous
   uint32_t magic;
   uint32_t shifts;
-  uint32_t kind;           // bits 0-7 kind, 8-15 element bytes, kRelSrcBuf / kRelDstBuf / kRelFar
+  uint32_t kind;           // bits 0-7 kind, 8-15 element bytes, kRelSrcBuf ... kRelShiftBit
   int32_t src_slot;        // index into the phase's pointer table, -1 = none
   int32_t dst_slot;
   int32_t dst2_slot;
@@ -914,10 +955,11 @@ __host__ __device__ __forceinline__ DevItem bind_item(const DevRel& h, const uin
   return d;
 }
 
-// Tile `j` of item `k` of `total` source bytes, bound as `item`.
-__host__ __device__ __forceinline__ DevTile tile_record(const DevItem& item, uint32_t k, uint32_t op, uint64_t total,
-                                                        uint32_t tile_shift, uint64_t j) {
-  const uint32_t width = item.row_bytes;
+// Tile `j` of item `k` with descriptor `h`, bound as `item`.
+__host__ __device__ __forceinline__ DevTile tile_record(const DevItem& item, const DevRel& h, uint32_t k, uint32_t op,
+                                                        uint64_t j) {
+  const uint32_t width = item.row_bytes, tile_shift = (h.kind >> kRelShiftBit) & 0x1fu;
+  const uint64_t total = h.total;
   uint64_t start = j << tile_shift;
   uint64_t n = total - start < (uint64_t(1) << tile_shift) ? total - start : (uint64_t(1) << tile_shift);
   if (width == 0 && total >= 16 && n < 16) {   // a whole vector, from the tile before
@@ -946,12 +988,11 @@ __host__ __device__ __forceinline__ DevTile tile_record(const DevItem& item, uin
 // chunk also writes the bound item.
 __global__ __launch_bounds__(kSetupBlock) void sr_tile_emit_kernel(
     const DevRel* __restrict__ rel, const uint64_t* __restrict__ tile_base, const EmitChunk* __restrict__ chunks,
-    uint32_t n_chunks, uint32_t tile_shift, DevTile* __restrict__ tiles, const uint64_t* __restrict__ ptrs,
+    uint32_t n_chunks, DevTile* __restrict__ tiles, const uint64_t* __restrict__ ptrs,
     const uint64_t* __restrict__ offset, DevItem* __restrict__ items) {
   for (uint32_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
     const uint32_t k = chunks[c].item;
     const uint64_t j0 = uint64_t(chunks[c].chunk) * kEmitTiles;
-    const uint64_t total = rel[k].total;
     const uint64_t cnt = tile_base[k + 1] - tile_base[k];
     // Items of a group have equal tile counts; tile j of member m goes to
     // group_start + j*M + m, so the members' tiles over the same rows are
@@ -964,7 +1005,7 @@ __global__ __launch_bounds__(kSetupBlock) void sr_tile_emit_kernel(
     if (j0 == 0 && threadIdx.x == 0) items[k] = item;
     const uint64_t j1 = cnt < j0 + kEmitTiles ? cnt : j0 + kEmitTiles;
     for (uint64_t j = j0 + threadIdx.x; j < j1; j += kSetupBlock) {
-      tiles[b + j * gsize] = tile_record(item, k, op, total, tile_shift, j);
+      tiles[b + j * gsize] = tile_record(item, rel[k], k, op, j);
     }
   }
 }
@@ -1004,6 +1045,7 @@ struct Phase {
   const char* src_name = "src_ptrs";    // caller-side names of the two tables
   const char* dst_name = "dst_ptrs";
   bool interleave = false;
+  Shape shape = kWide;
   uint64_t bytes_read = 0;
   uint64_t bytes_written = 0;
   // device state, created on first use: one device allocation carved into
@@ -1161,21 +1203,31 @@ uint32_t tile_reduce(const HostItem& h) {
   return (h.kind == kKindRecast && h.dst_slot >= 0) ? kRecastTileShift : 0;
 }
 
+// Source bytes of a tile record: what a workgroup moves in one pass, or
+// tile_bytes where that is more; for RECAST with an f32 copy the tile as plans
+// count it (16 MiB tiles of such rows: 911 us with twice as much, 692 so).
+uint32_t record_bytes(const HostItem& h, uint32_t tile_bytes) {
+  return std::max(tile_bytes >> tile_reduce(h), std::min(tile_bytes, kPassBytes));
+}
+
 // Whether a tile of a strided item may span 2 GiB or more of an object: its
 // rows are then addressed with 64-bit offsets.
-bool spans_far(const HostItem& h, uint32_t tile_bytes) {
-  const uint64_t rows = std::min<uint64_t>(h.rows, (uint64_t(tile_bytes) + h.row_bytes - 2) / h.row_bytes + 1);
+bool spans_far(const HostItem& h, uint32_t bytes) {
+  const uint64_t rows = std::min<uint64_t>(h.rows, (uint64_t(bytes) + h.row_bytes - 2) / h.row_bytes + 1);
   const uint64_t stride = std::max({h.src_stride, h.dst_stride, h.dst2_stride});
   return stride >= kNearBytes || rows * stride + h.row_bytes > kNearBytes;
 }
 
-void build_rel(Phase& ph, const std::vector<uint32_t>& order, uint32_t tile_bytes, bool buf_src,
-               bool buf_dst, bool group_by_src, bool row_groups) {
+void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_options& opt, bool buf_src,
+               bool buf_dst, bool group_by_src) {
+  const uint32_t tile_bytes = opt.tile_bytes;
+  const bool row_groups = !(opt.flags & SR_OPT_NO_ROW_GROUPS);
   ph.rel.clear();
   ph.rel.reserve(order.size());
   ph.tile_base.clear();
   ph.tile_base.reserve(order.size() + 1);
   ph.n_tiles = ph.n_recs = 0;
+  uint64_t total = 0;
   for (uint32_t k : order) {
     ph.tile_base.push_back(ph.n_recs);
     const HostItem& h = ph.items[k];
@@ -1198,7 +1250,9 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, uint32_t tile_byte
     r.kind = h.kind | (h.esize << 8);
     if (buf_src && h.src_slot >= 0) r.kind |= kRelSrcBuf;
     if (buf_dst && h.dst_slot >= 0) r.kind |= kRelDstBuf;
-    if (!h.contiguous && spans_far(h, tile_bytes)) r.kind |= kRelFar;
+    const uint32_t rec_bytes = record_bytes(h, tile_bytes);
+    r.kind |= log2u(rec_bytes) << kRelShiftBit;
+    if (!h.contiguous && spans_far(h, rec_bytes)) r.kind |= kRelFar;
     r.src_slot = h.src_slot;
     r.dst_slot = h.dst_slot >= 0 ? int32_t(ph.n_src_base) + h.dst_slot : -1;
     r.dst2_slot = h.dst2_slot >= 0 ? int32_t(ph.n_src_base) + h.dst2_slot : -1;
@@ -1212,9 +1266,11 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, uint32_t tile_byte
     ph.rel.push_back(r);
     const uint64_t item_tile = uint64_t(tile_bytes) >> tile_reduce(h);
     ph.n_tiles += (r.total + item_tile - 1) / item_tile;
-    ph.n_recs += (r.total + tile_bytes - 1) / tile_bytes;
+    ph.n_recs += (r.total + rec_bytes - 1) / rec_bytes;
+    total += r.total;
   }
   ph.tile_base.push_back(ph.n_recs);
+  if (ph.n_recs > 0) ph.shape = pick_shape(ph.n_recs, total, tile_bytes, opt.max_blocks);
   ph.emit_chunks.clear();
   for (size_t k = 0; k < ph.rel.size(); ++k) {
     const uint64_t cnt = ph.tile_base[k + 1] - ph.tile_base[k];
@@ -1238,7 +1294,7 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, uint32_t tile_byte
       const HostItem& b = ph.items[order[i]];
       const Side sa = side(a), sb = side(b);
       chain = !a.contiguous && !b.contiguous && a.kind == b.kind && a.rows == b.rows &&
-              a.row_bytes == b.row_bytes && sa.slot >= 0 && sa.slot == sb.slot &&
+              a.row_bytes == b.row_bytes && record_bytes(a, tile_bytes) == record_bytes(b, tile_bytes) && sa.slot >= 0 && sa.slot == sb.slot &&
               sa.stride == sb.stride && sb.off == sa.off + sa.width;
     }
     if (!chain) {
@@ -1466,8 +1522,7 @@ int setup_offsets(sr_plan* p, hipStream_t stream) {
 int emit_tables(sr_plan* p, Phase& ph, hipStream_t stream) {
   const uint32_t n_chunks = uint32_t(ph.emit_chunks.size());
   hipLaunchKernelGGL(sr_tile_emit_kernel, dim3(std::min<uint32_t>(n_chunks, 65535u)), dim3(kSetupBlock), 0, stream,
-                     ph.d_rel, ph.d_tile_base, ph.d_chunks, n_chunks, log2u(p->opt.tile_bytes), ph.d_tiles, ph.d_ptrs,
-                     p->d_offset, ph.d_items);
+                     ph.d_rel, ph.d_tile_base, ph.d_chunks, n_chunks, ph.d_tiles, ph.d_ptrs, p->d_offset, ph.d_items);
   SR_HIP_TRY(hipGetLastError());
   return SR_OK;
 }
@@ -1575,21 +1630,21 @@ int launch_copy(const sr_plan_options& opt, const Phase& ph, PhaseKind kind, con
   const uint32_t n_tiles = uint32_t(ph.n_recs);
   const uint32_t seg = ph.interleave ? (n_tiles + kXcds - 1) / kXcds : 0u;
   const uint32_t n_pos = seg ? seg * kXcds : n_tiles;
+  const uint32_t lanes = shape_lanes(ph.shape);
   uint32_t grid = n_pos;
   if (opt.max_blocks != 0) grid = std::min(grid, opt.max_blocks);
-  grid = std::min(grid, kMaxGrid);
+  grid = std::min(grid, 0xffffffffu / lanes);   // grid work-items stay below 2^32
   // A capped grid strides over the positions; a multiple of the segment
   // count keeps every segment on one die.
   if (seg && grid >= kXcds) grid -= grid % kXcds;
-  const bool nt = (opt.flags & SR_OPT_TEMPORAL) == 0;
   typedef void (*KernelFn)(const DevItem*, const DevTile*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t);
-  KernelFn fn;
-  switch (kind) {
-    case kPack: fn = nt ? sr_pack_kernel<true> : sr_pack_kernel<false>; break;
-    case kUnpack: fn = nt ? sr_unpack_kernel<true> : sr_unpack_kernel<false>; break;
-    default: fn = nt ? sr_gather_kernel<true> : sr_gather_kernel<false>; break;
-  }
-  hipLaunchKernelGGL(fn, dim3(grid), dim3(kBlock), 0, stream, items, tiles, n_tiles, seg, n_pos, grid,
+#define SR_PHASES(NT, B, U) {sr_pack_kernel<NT, B, U>, sr_unpack_kernel<NT, B, U>, sr_gather_kernel<NT, B, U>}
+#define SR_SHAPES(NT) {SR_PHASES(NT, 1024, 1), SR_PHASES(NT, 512, 2), SR_PHASES(NT, 256, 1), SR_PHASES(NT, 1024, 2)}
+  static const KernelFn kernels[2][4][3] = {SR_SHAPES(true), SR_SHAPES(false)};   // by Shape, PhaseKind
+#undef SR_SHAPES
+#undef SR_PHASES
+  const KernelFn fn = kernels[(opt.flags & SR_OPT_TEMPORAL) ? 1 : 0][ph.shape][kind];
+  hipLaunchKernelGGL(fn, dim3(grid), dim3(lanes), 0, stream, items, tiles, n_tiles, seg, n_pos, grid,
                      read_ahead ? n_tiles : 0u);
   SR_HIP_TRY(hipGetLastError());
   return SR_OK;
@@ -1621,7 +1676,6 @@ int run_small(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
     ph.bound_valid = ph.on_device = false;
     DevItem* items = reinterpret_cast<DevItem*>(table + o_items);
     DevTile* tiles = reinterpret_cast<DevTile*>(table + o_tiles);
-    const uint32_t tile_shift = log2u(p->opt.tile_bytes);
     for (uint32_t k = 0; k < n; ++k) {
       const DevRel& h = ph.rel[k];
       uint32_t op;
@@ -1629,7 +1683,7 @@ int run_small(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
       items[k] = item;
       const uint64_t cnt = ph.tile_base[k + 1] - ph.tile_base[k];
       DevTile* t = tiles + (ph.tile_base[k] - h.group_index * cnt + h.group_index);
-      for (uint64_t j = 0; j < cnt; ++j) t[j * h.group_size] = tile_record(item, k, op, h.total, tile_shift, j);
+      for (uint64_t j = 0; j < cnt; ++j) t[j * h.group_size] = tile_record(item, h, k, op, j);
     }
     ph.slot = slot;
     ph.bound = ptrs;
@@ -2162,15 +2216,13 @@ int sr_plan_create(const sr_tensor* src_tensors, int32_t n_src, const sr_tensor*
     p->unpack.n_dst_base = uint32_t(n_dst);
     p->gather.n_src_base = uint32_t(n_src);
     p->gather.n_dst_base = uint32_t(n_dst);
-    const bool groups = !(opt.flags & SR_OPT_NO_ROW_GROUPS);
     if (buffers) {
-      build_rel(p->pack, by_piece ? identity(p->pack.items.size()) : item_order(p->pack, true),
-                opt.tile_bytes, false, true, true, groups);
-      build_rel(p->unpack, by_piece ? identity(p->unpack.items.size()) : item_order(p->unpack, false),
-                opt.tile_bytes, true, false, false, groups);
+      build_rel(p->pack, by_piece ? identity(p->pack.items.size()) : item_order(p->pack, true), opt, false, true, true);
+      build_rel(p->unpack, by_piece ? identity(p->unpack.items.size()) : item_order(p->unpack, false), opt, true, false,
+                false);
     }
-    build_rel(p->gather, by_piece ? identity(p->gather.items.size()) : item_order(p->gather, false),
-              opt.tile_bytes, false, false, false, groups);
+    build_rel(p->gather, by_piece ? identity(p->gather.items.size()) : item_order(p->gather, false), opt, false, false,
+              false);
   }
   {
     // object sizes of each phase's pointer table, and the caller's names
@@ -2419,7 +2471,7 @@ int sr_gather_noalloc(const sr_plan* plan, const void* const* src_ptrs, void* co
   SR_HIP_TRY(hipMemcpyAsync(s, host.get(), up, hipMemcpyHostToDevice, stream));
   // gather items read no buffer offsets (no side is a peer buffer)
   hipLaunchKernelGGL(sr_tile_emit_kernel, dim3(std::min<uint32_t>(n_chunks, 65535u)), dim3(kSetupBlock), 0,
-                     stream, d_rel, d_base, d_chunks, n_chunks, log2u(plan->opt.tile_bytes), d_tiles, d_ptrs,
+                     stream, d_rel, d_base, d_chunks, n_chunks, d_tiles, d_ptrs,
                      static_cast<const uint64_t*>(nullptr), d_items);
   SR_HIP_TRY(hipGetLastError());
   return launch_copy(plan->opt, ph, kGather, d_items, d_tiles, true, stream);

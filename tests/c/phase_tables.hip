@@ -171,11 +171,11 @@ std::function<void()> body(const Launch& l, dim3 grid, dim3 block) {
     auto rel = l.arg<const DevRel*>(0);
     auto base = l.arg<const uint64_t*>(1);
     auto chunks = l.arg<const EmitChunk*>(2);
-    const uint32_t n_chunks = l.arg<uint32_t>(3), shift = l.arg<uint32_t>(4);
-    auto tiles = l.arg<DevTile*>(5);
-    auto ptrs = l.arg<const uint64_t*>(6);
-    auto offset = l.arg<const uint64_t*>(7);
-    auto items = l.arg<DevItem*>(8);
+    const uint32_t n_chunks = l.arg<uint32_t>(3);
+    auto tiles = l.arg<DevTile*>(4);
+    auto ptrs = l.arg<const uint64_t*>(5);
+    auto offset = l.arg<const uint64_t*>(6);
+    auto items = l.arg<DevItem*>(7);
     return [=] {
       for (uint32_t c = 0; c < n_chunks; ++c) {
         const DevRel& h = rel[chunks[c].item];
@@ -186,18 +186,22 @@ std::function<void()> body(const Launch& l, dim3 grid, dim3 block) {
         const uint64_t first = base[chunks[c].item] - h.group_index * cnt + h.group_index;
         const uint64_t j0 = uint64_t(chunks[c].chunk) * kEmitTiles;
         for (uint64_t j = j0; j < std::min<uint64_t>(cnt, j0 + kEmitTiles); ++j)
-          tiles[first + j * h.group_size] = tile_record(item, chunks[c].item, op, h.total, shift, j);
+          tiles[first + j * h.group_size] = tile_record(item, h, chunks[c].item, op, j);
       }
     };
   }
-  const std::set<const void*> copies = {
-      reinterpret_cast<const void*>(sr_pack_kernel<true>),    reinterpret_cast<const void*>(sr_pack_kernel<false>),
-      reinterpret_cast<const void*>(sr_unpack_kernel<true>),  reinterpret_cast<const void*>(sr_unpack_kernel<false>),
-      reinterpret_cast<const void*>(sr_gather_kernel<true>),  reinterpret_cast<const void*>(sr_gather_kernel<false>)};
+#define PHASES(NT, B, U)                                          \
+  reinterpret_cast<const void*>(sr_pack_kernel<NT, B, U>),        \
+      reinterpret_cast<const void*>(sr_unpack_kernel<NT, B, U>),  \
+      reinterpret_cast<const void*>(sr_gather_kernel<NT, B, U>)
+  static const std::set<const void*> copies = {PHASES(true, 1024, 1),  PHASES(true, 512, 2),  PHASES(true, 256, 1),
+                                               PHASES(true, 1024, 2),  PHASES(false, 1024, 1), PHASES(false, 512, 2),
+                                               PHASES(false, 256, 1), PHASES(false, 1024, 2)};
   if (copies.count(l.fn)) {
     auto items = l.arg<const DevItem*>(0);
     auto tiles = l.arg<const DevTile*>(1);
     const uint32_t n = l.arg<uint32_t>(2);
+    if (uint64_t(grid.x) * block.x > 0xffffffffu || n > l.arg<uint32_t>(4)) die("copy: grid");
     return [=, spans = writes] { copy_tiles(items, tiles, n, spans); };
   }
   die("unknown kernel");
@@ -400,12 +404,12 @@ struct Job {
   }
 };
 
-constexpr uint64_t kSmall = 64, kMost = kHostTableTiles, kLarge = kHostTableTiles + 40;
+constexpr uint64_t kFew = 64, kMost = kHostTableTiles, kMany = kHostTableTiles + 40;
 
 // Every route gives the same bytes: first, second and third launches of a
 // binding and returns to it, gather and pack + unpack.
 void routes() {
-  for (uint64_t tiles : {kSmall, kMost, kLarge})
+  for (uint64_t tiles : {kFew, kMost, kMany})
     for (uint64_t cols : {3, 16, 25, 64}) {
       Job j(tiles, 3, cols);
       for (int k : {0, 1, 2, 1, 1, 1, 0, 2, 2}) {
@@ -427,7 +431,7 @@ void routes() {
 // A first use on a capturing stream that fails after its table memory was
 // taken (from blocks that plans before it left), then the same calls again.
 void capture_fails() {
-  { Job before(kSmall, 1); ok(before.gather(0, 1), "gather"); ok(before.gather(0, 1), "gather"); drain({}); }
+  { Job before(kFew, 1); ok(before.gather(0, 1), "gather"); ok(before.gather(0, 1), "gather"); drain({}); }
   Job j(kMost, 1);
   model::streams[1].capturing = true;
   if (j.pack(0, 1) != SR_EHIP) die("a pack whose buffer offsets find no memory in a capture");
@@ -473,8 +477,8 @@ int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "routes") routes();
   else if (what == "capture_fails") capture_fails();
-  else if (what == "two_streams_small") for (int first : {1, 2, 3}) for (int n : {0, 1, 2}) two_streams(kSmall, first, n);
-  else if (what == "two_streams_large") for (int first : {1, 2, 3}) for (int n : {0, 1, 2}) two_streams(kLarge, first, n);
+  else if (what == "two_streams_small") for (int first : {1, 2, 3}) for (int n : {0, 1, 2}) two_streams(kFew, first, n);
+  else if (what == "two_streams_large") for (int first : {1, 2, 3}) for (int n : {0, 1, 2}) two_streams(kMany, first, n);
   else die("no such scenario");
   check_guards("end");
   std::puts("ok");

@@ -47,12 +47,12 @@ class Obj:
         assert bool((self.bytes[:lo] == POISON).all()) and bool((self.bytes[hi:] == POISON).all()), f"{what}: guard"
 
 
-def _gather(src, dst, pieces, tile_bytes=0, flags=0, noalloc=False):
+def _gather(src, dst, pieces, tile_bytes=0, flags=0, noalloc=False, max_blocks=0):
     L = _lib.lib()
     S = (_lib.SrTensor * max(1, len(src)))(*[_lib.SrTensor(o.rows, o.cols, DT[o.dt][0], 0) for o in src])
     D = (_lib.SrTensor * len(dst))(*[_lib.SrTensor(o.rows, o.cols, DT[o.dt][0], 0) for o in dst])
     P = (_lib.SrPiece * len(pieces))(*[_lib.SrPiece(*p) for p in pieces])
-    opt = _lib.SrPlanOptions(tile_bytes, 0, flags, 0)
+    opt = _lib.SrPlanOptions(tile_bytes, max_blocks, flags, 0)
     h = ctypes.c_void_p()
     _lib.check(L.sr_plan_create(S, len(src), D, len(dst), 1, P, len(pieces), ctypes.byref(opt), ctypes.byref(h)), "plan")
     try:
@@ -136,6 +136,32 @@ def test_recast_and_zero_rows(shift, flags):
         x.check(b.t[:, :c], c)
         y.check(b.t[:, :c].to(torch.bfloat16), c)
         n.check(torch.cat([a.t, b.t[:, :c]], 1).to(torch.bfloat16), c)
+
+
+@pytest.mark.parametrize("size,count,tile_bytes,max_blocks", [
+    (7168, 40, 0, 0), (7169, 40, 0, 0),             # mean bytes of a tile: 256 lanes up to 7 KiB,
+    (12288, 40, 0, 0), (12289, 40, 0, 0),           # 512 up to 12 KiB
+    (16384, 5120, 0, 0), (16384, 5121, 0, 0),       # 512 up to 5120 tiles, 1024 above
+    (16384, 6000, 0, 512), (16384, 6000, 0, 513),   # and for grids capped at 512
+    (100, 3000, 4096, 0), (90000, 300, 65536, 0), (90001, 300, 65536, 24), (65539, 7, 16384, 5)])
+def test_workgroups_by_tile_size(size, count, tile_bytes, max_blocks):
+    """`count` contiguous pieces of `size` bytes in reverse order, a band of
+    columns of as many bytes, split off and with both RECAST copies, beside
+    zeros: on both sides of each line where the workgroups change."""
+    print(f"[copy forms] {count} pieces of {size}, tile {tile_bytes}, {max_blocks} blocks", flush=True)
+    a, d = Obj(count, size, "u8", seed=size), Obj(count, size, "u8")
+    flat = [(COPY, 0, 0, 0, -1, 0, 1, size, count - 1 - k, 0, k, 0) for k in range(count)]
+    _gather([a], [d], flat, tile_bytes, max_blocks=max_blocks)
+    d.check(a.t.flip(0), "pieces")
+    rows, c = 64, max(1, size * count // 64 // 4)
+    b, x, y, h, z = (Obj(rows, 2 * c, "f32", seed=size + 1), Obj(rows, c, "f32"), Obj(rows, c, "f32"),
+                     Obj(rows, c, "bf16"), Obj(rows, c, "f32", 1))
+    _gather([b], [x, y, h, z], [copy(0, 0, rows, c), (RECAST, 0, 0, 1, 2, 0, rows, c, 0, c, 0, 0),
+                                (ZERO, 0, -1, 3, -1, 0, rows, c, 0, 0, 0, 0)], tile_bytes, max_blocks=max_blocks)
+    x.check(b.t[:, :c], "split")
+    y.check(b.t[:, c:], "recast: f32")
+    h.check(b.t[:, c:].to(torch.bfloat16), "recast: bf16")
+    z.check(torch.zeros_like(z.t), "zeros")
 
 
 def test_rows_two_gib_apart():
