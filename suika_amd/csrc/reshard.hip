@@ -425,16 +425,28 @@ __device__ __forceinline__ void put(const Regions& r, const Place& at, typename 
 // after them would hold the wave until they are written.  256 records cover a
 // die's tiles in flight twice over (flat copy of 2 GiB: 6.40 TB/s without,
 // 6.69 with 256 or 512 ahead, 6.47 with 2048).
+//
+// The same read takes the lines of the next 16 items along, for tiles that
+// need theirs: each new item's line otherwise stops all the tiles that are in
+// flight on a die (columns split off 64 tiles an item, 1024 items: 381 us
+// without, 328 with; 64 items 329 and 329).  One read for both, as a second
+// costs every such tile 10%.
 constexpr uint32_t kAhead = 256;
 constexpr uint32_t kAheadStep = 4;
+constexpr uint32_t kAheadItems = 16;
 
 struct Ahead {
   const DevTile* tiles;
   uint32_t i, n, lane;
+  const DevItem* items;
+  uint32_t item, n_items;   // item: n_items where a tile needs none
   template <int B>
   __device__ __forceinline__ void touch() const {
     if (lane >= B - 64 && i % kAheadStep == 0 && i + kAhead < n) {
-      const uint32_t x = __hip_atomic_load(&tiles[i + kAhead].info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      constexpr uint32_t kPerLine = 128 / sizeof(DevItem);
+      const uint32_t l = lane - (B - 64), k = item + l * kPerLine;
+      const uint32_t* at = l < kAheadItems / kPerLine && k < n_items ? &items[k].flags : &tiles[i + kAhead].info;
+      const uint32_t x = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       asm volatile("" ::"v"(x));
     }
   }
@@ -635,7 +647,7 @@ __device__ __forceinline__ void far_tile(const DevItem& it, const DevTile& t, ui
 template <bool NT, int B, int U>
 __device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, const DevTile* __restrict__ tiles,
                                            uint32_t n_tiles, uint32_t seg, uint32_t n_pos, uint32_t stride,
-                                           uint32_t n_ahead) {
+                                           uint32_t n_ahead, uint32_t n_items) {
   uint32_t p = blockIdx.x;
   do {
     const uint32_t i = seg ? (p % kXcds) * seg + p / kXcds : p;
@@ -645,8 +657,8 @@ __device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, co
       // be computed for all paths before the loop, and held
       uint32_t lane = threadIdx.x;
       asm volatile("" : "+v"(lane));
-      const Ahead ahead{tiles, i, n_ahead, lane};
       const uint32_t op = t.info >> kTileOpBit, nbytes = t.info & kTileBytesMask;
+      const Ahead ahead{tiles, i, n_ahead, lane, items, op == kOpCopy ? n_items : t.item, n_items};
       constexpr Policy kWhole = NT ? kThrough : kCached, kPartial = NT ? kStream : kCached;
       const Region none = region(0, 0);
       if (__builtin_expect(op == kOpCopy, 1)) {
@@ -700,8 +712,8 @@ __device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, co
   template <bool NT, int B, int U>                                                                           \
   __global__ __launch_bounds__(B) __attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(8))) void NAME(    \
       const DevItem* __restrict__ items, const DevTile* __restrict__ tiles, uint32_t n_tiles, uint32_t seg,  \
-      uint32_t n_pos, uint32_t stride, uint32_t n_ahead) {                                                   \
-    exec_tiles<NT, B, U>(items, tiles, n_tiles, seg, n_pos, stride, n_ahead);                                \
+      uint32_t n_pos, uint32_t stride, uint32_t n_ahead, uint32_t n_items) {                                 \
+    exec_tiles<NT, B, U>(items, tiles, n_tiles, seg, n_pos, stride, n_ahead, n_items);                       \
   }
 SR_COPY_KERNEL(sr_pack_kernel)
 SR_COPY_KERNEL(sr_unpack_kernel)
@@ -1637,7 +1649,7 @@ int launch_copy(const sr_plan_options& opt, const Phase& ph, PhaseKind kind, con
   // A capped grid strides over the positions; a multiple of the segment
   // count keeps every segment on one die.
   if (seg && grid >= kXcds) grid -= grid % kXcds;
-  typedef void (*KernelFn)(const DevItem*, const DevTile*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t);
+  typedef void (*KernelFn)(const DevItem*, const DevTile*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t);
 #define SR_PHASES(NT, B, U) {sr_pack_kernel<NT, B, U>, sr_unpack_kernel<NT, B, U>, sr_gather_kernel<NT, B, U>}
 #define SR_SHAPES(NT) {SR_PHASES(NT, 1024, 1), SR_PHASES(NT, 512, 2), SR_PHASES(NT, 256, 1), SR_PHASES(NT, 1024, 2)}
   static const KernelFn kernels[2][4][3] = {SR_SHAPES(true), SR_SHAPES(false)};   // by Shape, PhaseKind
@@ -1645,7 +1657,7 @@ int launch_copy(const sr_plan_options& opt, const Phase& ph, PhaseKind kind, con
 #undef SR_PHASES
   const KernelFn fn = kernels[(opt.flags & SR_OPT_TEMPORAL) ? 1 : 0][ph.shape][kind];
   hipLaunchKernelGGL(fn, dim3(grid), dim3(lanes), 0, stream, items, tiles, n_tiles, seg, n_pos, grid,
-                     read_ahead ? n_tiles : 0u);
+                     read_ahead ? n_tiles : 0u, uint32_t(ph.rel.size()));
   SR_HIP_TRY(hipGetLastError());
   return SR_OK;
 }

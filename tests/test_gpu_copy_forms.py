@@ -164,6 +164,21 @@ def test_workgroups_by_tile_size(size, count, tile_bytes, max_blocks):
     z.check(torch.zeros_like(z.t), "zeros")
 
 
+@pytest.mark.parametrize("bands,rows,tile_bytes", [(300, 256, 4096), (100, 4096, 0), (5, 40000, 0)])
+def test_items_read_ahead(bands, rows, tile_bytes):
+    """Bands of 64 columns, an item each, split off and merged again: tiles of
+    many items, of the last ones and of single items."""
+    print(f"[copy forms] {bands} bands of {rows} rows, tile {tile_bytes}", flush=True)
+    w = Obj(rows, 64 * bands, "f32", seed=bands)
+    parts = [Obj(rows, 64, "f32") for _ in range(bands)]
+    _gather([w], parts, [copy(0, k, rows, 64, sc=64 * k) for k in range(bands)], tile_bytes)
+    for k, p in enumerate(parts):
+        p.check(w.t[:, 64 * k:64 * k + 64], f"band {k}")
+    d = Obj(rows, 64 * bands, "f32")
+    _gather(parts, [d], [copy(k, 0, rows, 64, dc=64 * k) for k in range(bands)], tile_bytes)
+    d.check(w.t, "merged")
+
+
 def test_rows_two_gib_apart():
     """Rows so long that a tile's rows span 2 GiB: 64-bit offsets, beside a
     band of the same rows that is near enough within a smaller tile."""
