@@ -268,7 +268,8 @@ constexpr uint32_t kNowhere = 0xfffffff0u;
 // 7.5, nt 6.5).  Lines that several waves or rows write in parts are left for
 // the L2 to merge, as streaming lines or, for short rows, as ordinary ones
 // (side by side rows of 4 bytes: through 3.0 TB/s, nt 3.6, ordinary 5.1; of
-// 36 kB + 16 bytes: 5.4, 5.9, 5.5).
+// 36 kB + 16 bytes: 5.4, 5.9, 5.5).  Where whole lines are streamed all the
+// same: stream_whole.
 enum Policy : int {
   kCached = 0,
   kStream = 2,
@@ -741,11 +742,14 @@ enum Shape { kWide, kSmall, kTiny, kLong };
 
 constexpr uint32_t shape_lanes(Shape s) { return s == kSmall ? 512 : s == kTiny ? 256 : 1024; }
 
+constexpr uint64_t kFewTiles = 5120, kManyTiles = 16384;
+constexpr uint32_t kFewBlocks = 512;
+
 Shape pick_shape(uint64_t n_recs, uint64_t bytes, uint32_t tile_bytes, uint32_t max_blocks) {
   const uint64_t mean = bytes / n_recs;
   if (mean <= 7 * 1024) return kTiny;
   if (tile_bytes > kPassBytes) return kLong;
-  if (mean <= 12 * 1024 || n_recs <= 5120 || (max_blocks != 0 && max_blocks <= 512)) return kSmall;
+  if (mean <= 12 * 1024 || n_recs <= kFewTiles || (max_blocks != 0 && max_blocks <= kFewBlocks)) return kSmall;
   return kWide;
 }
 
@@ -764,6 +768,7 @@ enum : uint32_t {
   kRelSrcBuf = 1u << 16,   // source side is a peer buffer at the piece's offset
   kRelDstBuf = 1u << 17,   // destination side is a peer buffer at the piece's offset
   kRelFar = 1u << 18,      // kOpFar
+  kRelStream = 1u << 19,   // whole lines are streamed too (stream_whole)
   kRelShiftBit = 20,       // bits 20-24: log2 of the source bytes of a tile record
 };
 
@@ -954,14 +959,15 @@ __host__ __device__ __forceinline__ DevItem bind_item(const DevRel& h, const uin
   }
   const bool merge =
       !dense && (kind == kKindRecast || h.row_bytes < (kind == kKindZero ? kMergeZeroBelow : kMergeBelow));
-  const bool whole = (line & 63) == 0;
+  const bool whole = (line & 63) == 0, rows16 = !contiguous && h.row_bytes % 16 == 0;
+  const bool stream = (h.kind & kRelStream) != 0;
   if (far) op = kOpFar;
   else if (lv < 4 && (contiguous || merge || kind == kKindRecast || lv < 2)) op = kOpNarrow;
   else if (lv < 4) op = lv == 3 ? kOpRows8 : kOpRows4;
-  else if (contiguous && whole) op = kind == kKindCopy ? kOpCopy : kind == kKindZero ? kOpZero : kOpRecast;
+  else if (contiguous && whole && !stream) op = kind == kKindCopy ? kOpCopy : kind == kKindZero ? kOpZero : kOpRecast;
   else if (contiguous && kind == kKindCopy) op = kOpShifted;
-  else if (!contiguous && whole && h.row_bytes % 16 == 0) op = kind == kKindRecast ? kOpRecastRows : kOpRows;
-  else if (!contiguous && !merge && kind != kKindRecast && h.row_bytes % 16 == 0) op = kOpRowsPart;
+  else if (rows16 && whole && !stream) op = kind == kKindRecast ? kOpRecastRows : kOpRows;
+  else if (rows16 && kind != kKindRecast && (whole || !merge)) op = kOpRowsPart;
   else op = kOpWide;
   d.flags = kind | (lv << 4) | (merge ? kItemMerge : 0u);
   return d;
@@ -1230,6 +1236,28 @@ bool spans_far(const HostItem& h, uint32_t bytes) {
   return stride >= kNearBytes || rows * stride + h.row_bytes > kNearBytes;
 }
 
+// Whether an item's whole lines are streamed rather than written through the
+// L2 (Policy).  ZERO rows always are (1 GiB of rows of 1024 bytes 166 us,
+// through 201).  COPY lines written through are faster in large phases and in
+// those of few tiles (us, through / streamed: columns merged, 1500 tiles
+// 9.4 / 13.1, 40000 209 / 213; flat, 40000 tiles 200 / 203), but not
+//   * between, where much of the phase fits the memory-side cache (columns
+//     merged, 6000 tiles 36.5 / 35.7, 9000 53.2 / 51.6, 20000 108.7 / 108.8);
+//   * into rows that the launch does not write side by side from end to end
+//     (a band of wider rows, 9000 tiles 58.5 / 52.1, 80000 476 / 428);
+//   * where a workgroup goes on to other tiles and so waits for its stores:
+//     contiguous pieces under a capped grid or in tiles of several passes
+//     (1 GiB, 64 workgroups 1026 / 934, 1 MiB tiles 405 / 400).
+bool stream_whole(const HostItem& h, uint32_t group_size, const Phase& ph, const sr_plan_options& opt) {
+  if (h.kind != kKindCopy) return h.kind == kKindZero && !h.contiguous;
+  const bool loops = opt.tile_bytes > kPassBytes || (opt.max_blocks != 0 && opt.max_blocks <= kFewBlocks);
+  if (h.contiguous && loops) return true;
+  if (ph.n_recs <= kFewTiles) return false;
+  const bool side_by_side =
+      h.contiguous || h.dst_stride == h.row_bytes || h.dst_stride == h.row_bytes * group_size;
+  return !side_by_side || (ph.shape == kWide && ph.n_recs < kManyTiles);
+}
+
 void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_options& opt, bool buf_src,
                bool buf_dst, bool group_by_src) {
   const uint32_t tile_bytes = opt.tile_bytes;
@@ -1288,7 +1316,6 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
     const uint64_t cnt = ph.tile_base[k + 1] - ph.tile_base[k];
     for (uint64_t c = 0; c * kEmitTiles < cnt; ++c) ph.emit_chunks.push_back(EmitChunk{uint32_t(k), uint32_t(c)});
   }
-  if (!row_groups) return;
   struct Side {
     int64_t slot;
     uint64_t off, stride, width;
@@ -1301,7 +1328,7 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
   size_t first = 0;
   for (size_t i = 1; i <= order.size(); ++i) {
     bool chain = false;
-    if (i < order.size()) {
+    if (row_groups && i < order.size()) {
       const HostItem& a = ph.items[order[i - 1]];
       const HostItem& b = ph.items[order[i]];
       const Side sa = side(a), sb = side(b);
@@ -1314,6 +1341,7 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
       for (size_t g = first; g < i; ++g) {
         ph.rel[g].group_size = m;
         ph.rel[g].group_index = uint32_t(g - first);
+        if (stream_whole(ph.items[order[g]], m, ph, opt)) ph.rel[g].kind |= kRelStream;
       }
       first = i;
     }

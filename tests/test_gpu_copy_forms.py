@@ -179,6 +179,22 @@ def test_items_read_ahead(bands, rows, tile_bytes):
     d.check(w.t, "merged")
 
 
+@pytest.mark.parametrize("rows,tile_bytes", [(300, 0), (20400, 0), (20800, 0), (66000, 0), (1400, 65536)])
+def test_streamed_lines(rows, tile_bytes):
+    """A band of 1024 columns of wider rows beside a ZERO band, the rest of
+    the rows untouched, and whole rows, in phases of few tiles, of a middling
+    number (5121 to 16383) and of more."""
+    print(f"[copy forms] bands of {rows} rows, tile {tile_bytes}", flush=True)
+    a, d = Obj(rows, 1024, "f32", seed=rows), Obj(rows, 3072, "f32")
+    flat, e = Obj(1, 1024 * (rows // 8), "f32", seed=1), Obj(1, 1024 * (rows // 8), "f32")
+    _gather([a, flat], [d, e], [copy(0, 0, rows, 1024, dc=1024), (ZERO, 0, -1, 0, -1, 0, rows, 1024, 0, 0, 0, 2048),
+                                copy(1, 1, 1, flat.cols)], tile_bytes, flags=_lib.SR_OPT_SKIP_COVERAGE)
+    assert bool((d.t[:, :1024].contiguous().view(torch.uint8) == POISON).all()), "columns before the band"
+    d.t[:, :1024] = 0
+    d.check(torch.cat([torch.zeros_like(a.t), a.t, torch.zeros_like(a.t)], 1), "band")
+    e.check(flat.t, "whole rows")
+
+
 def test_rows_two_gib_apart():
     """Rows so long that a tile's rows span 2 GiB: 64-bit offsets, beside a
     band of the same rows that is near enough within a smaller tile."""
