@@ -733,7 +733,9 @@ SR_COPY_KERNEL(sr_gather_kernel)
 //   * few tiles, where each compute unit takes a handful in turn and more of
 //     them side by side hide the way to a tile's first load: 512 lanes of two
 //     vectors up to 5120 tiles (strided, 2624 tiles 18.2 / 15.7 us, 4000
-//     24.5 / 21.7, 6000 36.5 / 36.5);
+//     24.5 / 21.7, 6000 36.5 / 36.5), and up to 16384 where most are COPY
+//     rows, which then are streamed (1024 lanes of one / 512 of two: 8192
+//     tiles 50.8 / 49.1, 16384 91.8 / 89.1; contiguous ones 46.9 / 48.8);
 //   * grids capped at 512 workgroups or less, the same (1 GiB, 64 workgroups
 //     1123 / 1026 us, 256 421 / 378, 512 394 / 388);
 //   * tiles of more than one pass: two vectors in each of 1024 lanes (64 KiB
@@ -745,12 +747,18 @@ constexpr uint32_t shape_lanes(Shape s) { return s == kSmall ? 512 : s == kTiny 
 constexpr uint64_t kFewTiles = 5120, kManyTiles = 16384;
 constexpr uint32_t kFewBlocks = 512;
 
-Shape pick_shape(uint64_t n_recs, uint64_t bytes, uint32_t tile_bytes, uint32_t max_blocks) {
+// The phase's tiles number more than a few, but not many, and are large.
+bool middling(uint64_t n_recs, uint64_t bytes) {
+  return n_recs > kFewTiles && n_recs <= kManyTiles && bytes / n_recs > 12 * 1024;
+}
+
+// `row_recs`: the tiles of COPY rows.
+Shape pick_shape(uint64_t n_recs, uint64_t bytes, uint64_t row_recs, uint32_t tile_bytes, uint32_t max_blocks) {
   const uint64_t mean = bytes / n_recs;
   if (mean <= 7 * 1024) return kTiny;
   if (tile_bytes > kPassBytes) return kLong;
   if (mean <= 12 * 1024 || n_recs <= kFewTiles || (max_blocks != 0 && max_blocks <= kFewBlocks)) return kSmall;
-  return kWide;
+  return middling(n_recs, bytes) && 2 * row_recs > n_recs ? kSmall : kWide;
 }
 
 // ------------------------------------------------- device-side plan binding
@@ -1056,6 +1064,7 @@ struct Phase {
   std::vector<EmitChunk> emit_chunks;   // the emit kernel's work: every item's tiles in chunks
   uint64_t n_tiles = 0;                 // as the plan reports them
   uint64_t n_recs = 0;                  // tile records, one per workgroup: at most n_tiles
+  uint64_t rec_bytes = 0;               // their source bytes
   uint32_t n_src_base = 0;              // pointer table: sources, then destinations
   uint32_t n_dst_base = 0;
   std::vector<uint64_t> obj_bytes;      // per pointer-table slot: object size
@@ -1255,7 +1264,7 @@ bool stream_whole(const HostItem& h, uint32_t group_size, const Phase& ph, const
   if (ph.n_recs <= kFewTiles) return false;
   const bool side_by_side =
       h.contiguous || h.dst_stride == h.row_bytes || h.dst_stride == h.row_bytes * group_size;
-  return !side_by_side || (ph.shape == kWide && ph.n_recs < kManyTiles);
+  return !side_by_side || middling(ph.n_recs, ph.rec_bytes);
 }
 
 void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_options& opt, bool buf_src,
@@ -1266,8 +1275,8 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
   ph.rel.reserve(order.size());
   ph.tile_base.clear();
   ph.tile_base.reserve(order.size() + 1);
-  ph.n_tiles = ph.n_recs = 0;
-  uint64_t total = 0;
+  ph.n_tiles = ph.n_recs = ph.rec_bytes = 0;
+  uint64_t row_recs = 0;
   for (uint32_t k : order) {
     ph.tile_base.push_back(ph.n_recs);
     const HostItem& h = ph.items[k];
@@ -1306,11 +1315,13 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
     ph.rel.push_back(r);
     const uint64_t item_tile = uint64_t(tile_bytes) >> tile_reduce(h);
     ph.n_tiles += (r.total + item_tile - 1) / item_tile;
-    ph.n_recs += (r.total + rec_bytes - 1) / rec_bytes;
-    total += r.total;
+    const uint64_t recs = (r.total + rec_bytes - 1) / rec_bytes;
+    if (!h.contiguous && h.kind == kKindCopy) row_recs += recs;
+    ph.n_recs += recs;
+    ph.rec_bytes += r.total;
   }
   ph.tile_base.push_back(ph.n_recs);
-  if (ph.n_recs > 0) ph.shape = pick_shape(ph.n_recs, total, tile_bytes, opt.max_blocks);
+  if (ph.n_recs > 0) ph.shape = pick_shape(ph.n_recs, ph.rec_bytes, row_recs, tile_bytes, opt.max_blocks);
   ph.emit_chunks.clear();
   for (size_t k = 0; k < ph.rel.size(); ++k) {
     const uint64_t cnt = ph.tile_base[k + 1] - ph.tile_base[k];
