@@ -208,21 +208,25 @@ static_assert(sizeof(DevItem) == 64, "DevItem layout");
 
 constexpr uint32_t kItemMerge = 1u << 8;   // partly written lines are left to the L2 to merge
 
-// How a tile is moved.  The first five are the tiles of large tensors; "rows"
-// are strided.  ZERO rows are copied from a source of no bytes.
+// How a tile is moved; "rows" are strided.  ZERO rows are copied from a source
+// of no bytes.  The first seven are the tiles of large tensors; of those the
+// first five write whole lines through.
 enum : uint32_t {
-  kOpCopy = 0,         // contiguous, whole lines written through
-  kOpRows = 1,         // rows of a multiple of 16 bytes, whole lines written through
-  kOpRecast = 2,       // contiguous f32 -> f32 copy (where there is one) + bf16 copy
-  kOpZero = 3,
-  kOpRecastRows = 4,
-  kOpShifted = 5,      // contiguous copy into parts of lines, streamed
-  kOpRowsPart = 6,     // rows of a multiple of 16 bytes, streamed
-  kOpRows8 = 7,        // rows copied in 8-byte vectors, streamed
+  kOpCopy = 0,           // contiguous
+  kOpRows = 1,           // COPY and ZERO rows of a multiple of 16 bytes
+  kOpRecast = 2,         // contiguous f32 -> f32 copy (where there is one) + bf16 copy
+  kOpZero = 3,           // contiguous
+  kOpRecastRows = 4,     // rows of a multiple of 16 bytes
+  kOpCopyStream = 5,     // kOpCopy, streamed
+  kOpRowsStream = 6,     // kOpRows, streamed
+  kOpRows8 = 7,          // COPY rows in 8-byte vectors, streamed
   kOpRows4 = 8,
-  kOpNarrow = 9,       // vectors of less than 16 bytes otherwise
-  kOpWide = 10,        // 16-byte vectors otherwise
-  kOpFar = 11,         // rows 2 GiB or more apart
+  kOpWide = 9,           // COPY and ZERO rows of other widths, in 16-byte vectors
+  kOpNarrow = 10,        // vectors of less than 16 bytes otherwise
+  kOpRecastRowsPart = 11,   // kOpRecastRows, streamed or left to the L2
+  kOpRecastStream = 12,     // kOpRecast, streamed
+  kOpZeroStream = 13,       // kOpZero, streamed
+  kOpFar = 14,           // rows 2 GiB or more apart
 };
 
 // The record of one tile.  A contiguous COPY or ZERO tile needs nothing else.
@@ -456,7 +460,7 @@ struct Ahead {
 // A tile of at least 16 contiguous bytes, at any alignment: 16 bytes per
 // lane, the last vector moved back to end with the tile (it then writes
 // bytes of its neighbour again, with the same values).
-template <uint32_t KIND, bool NT, Policy POLICY, int B, int U>
+template <uint32_t KIND, Policy POLICY, bool NT, int B, int U>
 __device__ __forceinline__ void contiguous_tile(const Regions& r, uint32_t nbytes, const Ahead& ahead) {
   for (uint32_t base = 0; base < nbytes; base += B * U * 16) {
     uint32_t off[U];
@@ -469,12 +473,12 @@ __device__ __forceinline__ void contiguous_tile(const Regions& r, uint32_t nbyte
     }
     if (KIND != kKindZero && base == 0) ahead.touch<B>();
 #pragma unroll
-    for (int u = 0; u < U; ++u) put<KIND, 16, POLICY>(r, Place{off[u], off[u], off[u] >> 1}, v[u]);
+    for (int u = 0; u < U; ++u) put<KIND, 16, NT ? POLICY : kCached>(r, Place{off[u], off[u], off[u] >> 1}, v[u]);
   }
 }
 
 // A tile of rows of a multiple of 16 bytes, at any alignment: 16 bytes per lane.
-template <uint32_t KIND, bool NT, Policy POLICY, int B, int U>
+template <uint32_t KIND, Policy POLICY, bool NT, int B, int U>
 __device__ __forceinline__ void rows_tile(const Regions& r, const DevItem& it, uint32_t column, uint32_t nbytes,
                                           const Ahead& ahead) {
   const RowMap rows = row_map(it, column);
@@ -493,18 +497,9 @@ __device__ __forceinline__ void rows_tile(const Regions& r, const DevItem& it, u
     }
     if (base == 0) ahead.touch<B>();
 #pragma unroll
-    for (int u = 0; u < U; ++u) put<KIND, 16, POLICY>(r, at[u], v[u]);
+    for (int u = 0; u < U; ++u) put<KIND, 16, NT ? POLICY : kCached>(r, at[u], v[u]);
   }
 }
-
-// The forms below branch at run time where that saves code: with a variant
-// of every form for every kind and policy the kernel grew from 20 to 46 KB,
-// and the paths above lost 3% to its instruction fetches.
-#define SR_BY_POLICY(MERGE, CALL)       \
-  do {                                  \
-    if (NT && !(MERGE)) CALL(kStream);  \
-    else CALL(kCached);                 \
-  } while (0)
 
 // The regions of a strided tile (or of a contiguous piece that is one tile,
 // from its origin).
@@ -514,62 +509,51 @@ __device__ __forceinline__ Regions row_regions(const DevItem& it, uint64_t row) 
           region(it.dst2 + row * it.dst2_stride, it.dst2 ? kNearBytes : 0)};
 }
 
-// 16-byte vectors at any alignment, rows of at least 16 bytes.  A vector
-// that runs over the end of its row (rows that are no multiple of 16 bytes;
-// not RECAST) becomes two, the last 16 bytes of that row and the first 16 of
-// the next; the bytes that neighbouring lanes write too have the same values.
-template <bool NT, int B>
+// The regions of a contiguous RECAST tile.
+__device__ __forceinline__ Regions recast_regions(const DevItem& it, const DevTile& t, uint32_t nbytes) {
+  return {region(t.src, nbytes), region(t.dst, t.dst ? nbytes : 0),
+          region(it.dst2 + ((t.src - it.src) >> 1), nbytes >> 1)};
+}
+
+// COPY and ZERO rows of at least 16 bytes at any alignment, in 16-byte vectors.
+// A vector that runs over the end of its row becomes two, the last 16 bytes of
+// that row and the first 16 of the next; the bytes that neighbouring lanes
+// write too have the same values.
+template <Policy POLICY, bool NT, int B>
 __device__ __forceinline__ void wide_tile(const DevItem& it, const DevTile& t, uint32_t nbytes, const Ahead& ahead) {
-  const bool strided = it.row_bytes != 0, recast = (it.flags & 0xfu) == kKindRecast;
-  const Regions r = strided ? row_regions(it, t.src)
-                            : Regions{region(t.src, it.src ? nbytes : 0), region(t.dst, t.dst ? nbytes : 0),
-                                      region(it.dst2 + ((t.src - it.src) >> 1), it.dst2 ? nbytes >> 1 : 0)};
+  const Regions r = row_regions(it, t.src);
   const RowMap rows = row_map(it, uint32_t(t.dst));
-  const uint32_t ss = uint32_t(it.src_stride), ds = uint32_t(it.dst_stride), hs = uint32_t(it.dst2_stride);
+  const uint32_t ss = uint32_t(it.src_stride), ds = uint32_t(it.dst_stride);
   for (uint32_t base = 0; base < nbytes; base += B * 16) {
-    const uint32_t b = base + ahead.lane * 16;
-    Place at, at2{kNowhere, kNowhere, kNowhere};
-    if (strided) {
-      const RowVec x = row_vec(rows, b, nbytes);
-      if (x.in) at = {x.row * ss + x.col, x.row * ds + x.col, x.row * hs + (x.col >> 1)};
-      else at = at2;
-      if (x.next) at2 = {(x.row + 1) * ss, (x.row + 1) * ds, kNowhere};
-    } else {
-      const uint32_t off = contiguous_vec(b, nbytes);
-      at = {off, off, off >> 1};
-    }
-    const VecOf<16>::type v = ld<16, NT>(r.src, at.src), w = ld<16, NT>(r.src, at2.src);
-    const VecOf<8>::type h = to_bf16<4>(v);
+    const RowVec x = row_vec(rows, base + ahead.lane * 16, nbytes);
+    const uint32_t from = x.in ? x.row * ss + x.col : kNowhere, to = x.in ? x.row * ds + x.col : kNowhere;
+    const uint32_t from2 = x.next ? (x.row + 1) * ss : kNowhere, to2 = x.next ? (x.row + 1) * ds : kNowhere;
+    const VecOf<16>::type v = ld<16, NT>(r.src, from), w = ld<16, NT>(r.src, from2);
     if (base == 0) ahead.touch<B>();
-#define SR_PUT(POLICY)                                \
-  do {                                                \
-    st<16, POLICY>(r.dst, at.dst, v);                 \
-    if (recast) st<8, POLICY>(r.half, at.half, h);    \
-    else st<16, POLICY>(r.dst, at2.dst, w);           \
-  } while (0)
-    SR_BY_POLICY(it.flags & kItemMerge, SR_PUT);
-#undef SR_PUT
+    st<16, NT ? POLICY : kCached>(r.dst, to, v);
+    st<16, NT ? POLICY : kCached>(r.dst, to2, w);
   }
 }
 
 // Vectors of the widest aligned type that divides the rows (RECAST: one
-// element).  A wave takes consecutive bytes, U vectors per lane a wave's
+// element).  A wave takes consecutive bytes, W vectors per lane a wave's
 // width apart: each vector's lines are then written by one wave (side by
 // side f32 rows of 16396 bytes: 5.7 TB/s, with the vectors of a lane a
 // workgroup's width apart 5.2).
-template <uint32_t KIND, int VB, bool NT, Policy POLICY, int B>
-__device__ __forceinline__ void narrow_vectors(const Regions& r, const DevItem& it, uint32_t column, uint32_t nbytes,
-                                               const Ahead& ahead) {
-  constexpr int U = VB == 8 ? 2 : 4;
+template <uint32_t KIND, int VB, Policy POLICY, bool NT, int B>
+__device__ __forceinline__ void narrow_tile(const DevItem& it, const DevTile& t, uint32_t nbytes, const Ahead& ahead) {
+  constexpr int W = VB == 8 ? 2 : 4;
   constexpr uint32_t kStep = 64 * VB;
-  const RowMap rows = row_map(it, column);
-  for (uint32_t base = 0; base < nbytes; base += B * VB * U) {
-    uint32_t b = base + (ahead.lane >> 6) * (U * kStep) + (ahead.lane & 63) * VB;
+  const bool strided = it.row_bytes != 0;
+  const Regions r = row_regions(it, strided ? t.src : 0);
+  const RowMap rows = row_map(it, strided ? uint32_t(t.dst) : 0);
+  for (uint32_t base = 0; base < nbytes; base += B * VB * W) {
+    uint32_t b = base + (ahead.lane >> 6) * (W * kStep) + (ahead.lane & 63) * VB;
     RowWalk walk(rows, b, kStep, uint32_t(it.src_stride), uint32_t(it.dst_stride), uint32_t(it.dst2_stride));
-    Place at[U];
-    typename VecOf<VB>::type v[U];
+    Place at[W];
+    typename VecOf<VB>::type v[W];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int u = 0; u < W; ++u) {
       const bool in = b < nbytes;
       at[u] = {kNowhere, in ? walk.at.dst : kNowhere, in ? walk.at.half : kNowhere};
       v[u] = ld<VB, NT>(r.src, in ? walk.at.src : kNowhere);
@@ -578,29 +562,30 @@ __device__ __forceinline__ void narrow_vectors(const Regions& r, const DevItem& 
     }
     if (base == 0) ahead.touch<B>();
 #pragma unroll
-    for (int u = 0; u < U; ++u) put<KIND, VB, POLICY>(r, at[u], v[u]);
+    for (int u = 0; u < W; ++u) put<KIND, VB, NT ? POLICY : kCached>(r, at[u], v[u]);
   }
 }
 
+// kOpNarrow.  A body for each policy here and above: one that branches before
+// its stores is 10% slower (rows of 17 bytes 458 us, so 398; of 2 bytes 319 /
+// 290), and large shares 0.4% where their forms branch.
 template <bool NT, int B>
-__device__ __forceinline__ void narrow_tile(const DevItem& it, const DevTile& t, uint32_t nbytes, const Ahead& ahead) {
-  const bool strided = it.row_bytes != 0, merge = !NT || (it.flags & kItemMerge);
-  const uint32_t lv = (it.flags >> 4) & 0xfu, column = strided ? uint32_t(t.dst) : 0;
-  const Regions r = row_regions(it, strided ? t.src : 0);
-  constexpr Policy kPart = NT ? kStream : kCached;
+__device__ __forceinline__ void narrow_forms(const DevItem& it, const DevTile& t, uint32_t nbytes, const Ahead& ahead) {
+  const uint32_t lv = (it.flags >> 4) & 0xfu;
+  const bool merge = it.flags & kItemMerge;
   if ((it.flags & 0xfu) == kKindRecast) {
-    if (merge) narrow_vectors<kKindRecast, 4, NT, kCached, B>(r, it, column, nbytes, ahead);
-    else narrow_vectors<kKindRecast, 4, NT, kPart, B>(r, it, column, nbytes, ahead);
+    if (merge) narrow_tile<kKindRecast, 4, kCached, NT, B>(it, t, nbytes, ahead);
+    else narrow_tile<kKindRecast, 4, kStream, NT, B>(it, t, nbytes, ahead);
   } else if (lv == 3) {   // streamed: kOpRows8, kOpRows4, or one small piece
-    narrow_vectors<kKindCopy, 8, NT, kCached, B>(r, it, column, nbytes, ahead);
+    narrow_tile<kKindCopy, 8, kCached, NT, B>(it, t, nbytes, ahead);
   } else if (lv == 2) {
-    narrow_vectors<kKindCopy, 4, NT, kCached, B>(r, it, column, nbytes, ahead);
+    narrow_tile<kKindCopy, 4, kCached, NT, B>(it, t, nbytes, ahead);
   } else if (lv == 1) {
-    if (merge) narrow_vectors<kKindCopy, 2, NT, kCached, B>(r, it, column, nbytes, ahead);
-    else narrow_vectors<kKindCopy, 2, NT, kPart, B>(r, it, column, nbytes, ahead);
+    if (merge) narrow_tile<kKindCopy, 2, kCached, NT, B>(it, t, nbytes, ahead);
+    else narrow_tile<kKindCopy, 2, kStream, NT, B>(it, t, nbytes, ahead);
   } else {
-    if (merge) narrow_vectors<kKindCopy, 1, NT, kCached, B>(r, it, column, nbytes, ahead);
-    else narrow_vectors<kKindCopy, 1, NT, kPart, B>(r, it, column, nbytes, ahead);
+    if (merge) narrow_tile<kKindCopy, 1, kCached, NT, B>(it, t, nbytes, ahead);
+    else narrow_tile<kKindCopy, 1, kStream, NT, B>(it, t, nbytes, ahead);
   }
 }
 
@@ -660,43 +645,49 @@ __device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, co
       asm volatile("" : "+v"(lane));
       const uint32_t op = t.info >> kTileOpBit, nbytes = t.info & kTileBytesMask;
       const Ahead ahead{tiles, i, n_ahead, lane, items, op == kOpCopy ? n_items : t.item, n_items};
-      constexpr Policy kWhole = NT ? kThrough : kCached, kPartial = NT ? kStream : kCached;
       const Region none = region(0, 0);
       if (__builtin_expect(op == kOpCopy, 1)) {
-        contiguous_tile<kKindCopy, NT, kWhole, B, U>(Regions{region(t.src, nbytes), region(t.dst, nbytes), none},
-                                                     nbytes, ahead);
+        contiguous_tile<kKindCopy, kThrough, NT, B, U>(Regions{region(t.src, nbytes), region(t.dst, nbytes), none},
+                                                       nbytes, ahead);
       } else if (__builtin_expect(op == kOpRows, 1)) {
         const DevItem it = items[t.item];
-        rows_tile<kKindCopy, NT, kWhole, B, U>(
+        rows_tile<kKindCopy, kThrough, NT, B, U>(
             Regions{region(it.src + t.src * it.src_stride, it.src ? kNearBytes : 0),
                     region(it.dst + t.src * it.dst_stride, kNearBytes), none},
             it, uint32_t(t.dst), nbytes, ahead);
       } else if (__builtin_expect(op == kOpRecast, 1)) {
-        const uint64_t half = items[t.item].dst2 + ((t.src - items[t.item].src) >> 1);
-        contiguous_tile<kKindRecast, NT, kWhole, B, U>(
-            Regions{region(t.src, nbytes), region(t.dst, t.dst ? nbytes : 0), region(half, nbytes >> 1)}, nbytes,
-            ahead);
+        contiguous_tile<kKindRecast, kThrough, NT, B, U>(recast_regions(items[t.item], t, nbytes), nbytes, ahead);
       } else if (__builtin_expect(op == kOpZero, 1)) {
-        contiguous_tile<kKindZero, NT, kWhole, B, U>(Regions{none, region(t.dst, nbytes), none}, nbytes, ahead);
+        contiguous_tile<kKindZero, kThrough, NT, B, U>(Regions{none, region(t.dst, nbytes), none}, nbytes, ahead);
       } else if (__builtin_expect(op == kOpRecastRows, 1)) {
         const DevItem it = items[t.item];
-        rows_tile<kKindRecast, NT, kWhole, B, U>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
-      } else if (op == kOpShifted) {
-        contiguous_tile<kKindCopy, NT, kPartial, B, U>(Regions{region(t.src, nbytes), region(t.dst, nbytes), none},
-                                                       nbytes, ahead);
-      } else if (op == kOpRowsPart) {
+        rows_tile<kKindRecast, kThrough, NT, B, U>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
+      } else if (op == kOpCopyStream) {
+        contiguous_tile<kKindCopy, kStream, NT, B, U>(Regions{region(t.src, nbytes), region(t.dst, nbytes), none},
+                                                      nbytes, ahead);
+      } else if (op == kOpRowsStream) {
         const DevItem it = items[t.item];
-        rows_tile<kKindCopy, NT, kPartial, B, U>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
+        rows_tile<kKindCopy, kStream, NT, B, U>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
       } else if (op == kOpRows8) {
-        const DevItem it = items[t.item];
-        narrow_vectors<kKindCopy, 8, NT, kPartial, B>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
+        narrow_tile<kKindCopy, 8, kStream, NT, B>(items[t.item], t, nbytes, ahead);
       } else if (op == kOpRows4) {
-        const DevItem it = items[t.item];
-        narrow_vectors<kKindCopy, 4, NT, kPartial, B>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
-      } else if (op == kOpNarrow) {
-        narrow_tile<NT, B>(items[t.item], t, nbytes, ahead);
+        narrow_tile<kKindCopy, 4, kStream, NT, B>(items[t.item], t, nbytes, ahead);
       } else if (op == kOpWide) {
-        wide_tile<NT, B>(items[t.item], t, nbytes, ahead);
+        const DevItem it = items[t.item];
+        if (it.flags & kItemMerge) wide_tile<kCached, NT, B>(it, t, nbytes, ahead);
+        else wide_tile<kStream, NT, B>(it, t, nbytes, ahead);
+      } else if (op == kOpNarrow) {
+        const DevItem it = items[t.item];
+        narrow_forms<NT, B>(it, t, nbytes, ahead);
+      } else if (op == kOpRecastRowsPart) {
+        const DevItem it = items[t.item];
+        const Regions r = row_regions(it, t.src);
+        if (it.flags & kItemMerge) rows_tile<kKindRecast, kCached, NT, B, U>(r, it, uint32_t(t.dst), nbytes, ahead);
+        else rows_tile<kKindRecast, kStream, NT, B, U>(r, it, uint32_t(t.dst), nbytes, ahead);
+      } else if (op == kOpRecastStream) {
+        contiguous_tile<kKindRecast, kStream, NT, B, U>(recast_regions(items[t.item], t, nbytes), nbytes, ahead);
+      } else if (op == kOpZeroStream) {
+        contiguous_tile<kKindZero, kStream, NT, B, U>(Regions{none, region(t.dst, nbytes), none}, nbytes, ahead);
       } else {
         far_tile<B>(items[t.item], t, nbytes, lane);
       }
@@ -752,7 +743,8 @@ bool middling(uint64_t n_recs, uint64_t bytes) {
   return n_recs > kFewTiles && n_recs <= kManyTiles && bytes / n_recs > 12 * 1024;
 }
 
-// `row_recs`: the tiles of COPY rows.
+// `row_recs`: the tiles of COPY rows of 512 bytes and more and of a multiple of
+// 16 (of 16 bytes, 16384 tiles: 117 us with 1024 lanes, 132 with 512).
 Shape pick_shape(uint64_t n_recs, uint64_t bytes, uint64_t row_recs, uint32_t tile_bytes, uint32_t max_blocks) {
   const uint64_t mean = bytes / n_recs;
   if (mean <= 7 * 1024) return kTiny;
@@ -918,9 +910,11 @@ __host__ __device__ inline uint32_t ragged_from(uint32_t vb, bool dense) {
 }
 
 // Rows of a destination that is not dense leave their lines to be merged
-// when they are shorter than this, RECAST at any width: f32 rows of 260 bytes
-// streamed 4.4, merged 4.9 TB/s; of 800 bytes 5.7 / 5.5; ZERO rows of 192
-// bytes 2.9 / 3.5, of 400 bytes 4.7 / 3.5; RECAST of 800 bytes 5.3 / 5.6.
+// when they are shorter than this, RECAST with an f32 copy or in single
+// elements at any width: f32 rows of 260 bytes streamed 4.4, merged 4.9 TB/s;
+// of 800 bytes 5.7 / 5.5; ZERO rows of 192 bytes 2.9 / 3.5, of 400 bytes 4.7 /
+// 3.5; RECAST of 800 bytes 5.1 / 6.0, of 16400 bytes 5.7 / 6.0, into bf16 alone
+// of 400 bytes 5.8 / 6.0, of 1600 bytes 6.3 / 5.9.
 constexpr uint32_t kMergeBelow = 512, kMergeZeroBelow = 384;
 
 // The item of descriptor `h`: its object addresses resolved from `ptrs`,
@@ -965,19 +959,20 @@ __host__ __device__ __forceinline__ DevItem bind_item(const DevRel& h, const uin
     line |= h.row_bytes | h.dst_stride | h.dst2_stride;
     if (kind == kKindRecast) line |= h.row_bytes >> 1;
   }
-  const bool merge =
-      !dense && (kind == kKindRecast || h.row_bytes < (kind == kKindZero ? kMergeZeroBelow : kMergeBelow));
   const bool whole = (line & 63) == 0, rows16 = !contiguous && h.row_bytes % 16 == 0;
-  const bool stream = (h.kind & kRelStream) != 0;
+  const bool merge = !dense && (kind == kKindRecast ? lv < 4 || h.dst_slot >= 0 || h.row_bytes < kMergeBelow
+                                                    : h.row_bytes < (kind == kKindZero ? kMergeZeroBelow : kMergeBelow));
+  const bool through = whole && !(h.kind & kRelStream);
   if (far) op = kOpFar;
   else if (lv < 4 && (contiguous || merge || kind == kKindRecast || lv < 2)) op = kOpNarrow;
   else if (lv < 4) op = lv == 3 ? kOpRows8 : kOpRows4;
-  else if (contiguous && whole && !stream) op = kind == kKindCopy ? kOpCopy : kind == kKindZero ? kOpZero : kOpRecast;
-  else if (contiguous && kind == kKindCopy) op = kOpShifted;
-  else if (rows16 && whole && !stream) op = kind == kKindRecast ? kOpRecastRows : kOpRows;
-  else if (rows16 && kind != kKindRecast && (whole || !merge)) op = kOpRowsPart;
+  else if (contiguous && through) op = kind == kKindCopy ? kOpCopy : kind == kKindZero ? kOpZero : kOpRecast;
+  else if (contiguous) op = kind == kKindCopy ? kOpCopyStream : kind == kKindZero ? kOpZeroStream : kOpRecastStream;
+  else if (kind == kKindRecast) op = through ? kOpRecastRows : kOpRecastRowsPart;
+  else if (rows16 && through) op = kOpRows;
+  else if (rows16 && (whole || !merge)) op = kOpRowsStream;
   else op = kOpWide;
-  d.flags = kind | (lv << 4) | (merge ? kItemMerge : 0u);
+  d.flags = kind | (lv << 4) | (merge && !whole ? kItemMerge : 0u);
   return d;
 }
 
@@ -1233,7 +1228,12 @@ uint32_t tile_reduce(const HostItem& h) {
 // Source bytes of a tile record: what a workgroup moves in one pass, or
 // tile_bytes where that is more; for RECAST with an f32 copy the tile as plans
 // count it (16 MiB tiles of such rows: 911 us with twice as much, 692 so).
-uint32_t record_bytes(const HostItem& h, uint32_t tile_bytes) {
+// RECAST into bf16 alone moves 1.5 x its source bytes, and a tile of it too
+// little for its start: two passes, except in phases of `few` tiles (rows of
+// 16 KiB split off 139 us with one, 123 with two; merged 278 / 244; rows of
+// 2732 bytes merged 359 / 285).
+uint32_t record_bytes(const HostItem& h, uint32_t tile_bytes, bool few) {
+  if (h.kind == kKindRecast && h.dst_slot < 0 && tile_bytes <= kPassBytes && !few) return tile_bytes * 2;
   return std::max(tile_bytes >> tile_reduce(h), std::min(tile_bytes, kPassBytes));
 }
 
@@ -1247,23 +1247,25 @@ bool spans_far(const HostItem& h, uint32_t bytes) {
 
 // Whether an item's whole lines are streamed rather than written through the
 // L2 (Policy).  ZERO rows always are (1 GiB of rows of 1024 bytes 166 us,
-// through 201).  COPY lines written through are faster in large phases and in
+// through 201).  Others written through are faster in large phases and in
 // those of few tiles (us, through / streamed: columns merged, 1500 tiles
 // 9.4 / 13.1, 40000 209 / 213; flat, 40000 tiles 200 / 203), but not
-//   * between, where much of the phase fits the memory-side cache (columns
-//     merged, 6000 tiles 36.5 / 35.7, 9000 53.2 / 51.6, 20000 108.7 / 108.8);
+//   * between, where much of the phase fits the memory-side cache, for rows
+//     and RECAST (columns merged, 6000 tiles 36.5 / 35.7, 9000 53.2 / 51.6,
+//     20000 108.7 / 108.8; RECAST, merged, 6000 tiles 46.2 / 43.2, 40000
+//     264.8 / 267.1);
 //   * into rows that the launch does not write side by side from end to end
 //     (a band of wider rows, 9000 tiles 58.5 / 52.1, 80000 476 / 428);
 //   * where a workgroup goes on to other tiles and so waits for its stores:
 //     contiguous pieces under a capped grid or in tiles of several passes
 //     (1 GiB, 64 workgroups 1026 / 934, 1 MiB tiles 405 / 400).
 bool stream_whole(const HostItem& h, uint32_t group_size, const Phase& ph, const sr_plan_options& opt) {
-  if (h.kind != kKindCopy) return h.kind == kKindZero && !h.contiguous;
+  if (h.kind == kKindZero) return !h.contiguous;
+  if (h.kind == kKindRecast) return h.dst_slot >= 0 && middling(ph.n_recs, ph.rec_bytes);
   const bool loops = opt.tile_bytes > kPassBytes || (opt.max_blocks != 0 && opt.max_blocks <= kFewBlocks);
   if (h.contiguous && loops) return true;
-  if (ph.n_recs <= kFewTiles) return false;
-  const bool side_by_side =
-      h.contiguous || h.dst_stride == h.row_bytes || h.dst_stride == h.row_bytes * group_size;
+  if (h.contiguous || ph.n_recs <= kFewTiles) return false;
+  const bool side_by_side = h.dst_stride == h.row_bytes || h.dst_stride == h.row_bytes * group_size;
   return !side_by_side || middling(ph.n_recs, ph.rec_bytes);
 }
 
@@ -1276,7 +1278,9 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
   ph.tile_base.clear();
   ph.tile_base.reserve(order.size() + 1);
   ph.n_tiles = ph.n_recs = ph.rec_bytes = 0;
-  uint64_t row_recs = 0;
+  uint64_t row_recs = 0, all_bytes = 0;
+  for (const HostItem& h : ph.items) all_bytes += h.rows * h.row_bytes;
+  const bool few = all_bytes / tile_bytes <= kFewTiles;
   for (uint32_t k : order) {
     ph.tile_base.push_back(ph.n_recs);
     const HostItem& h = ph.items[k];
@@ -1299,7 +1303,7 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
     r.kind = h.kind | (h.esize << 8);
     if (buf_src && h.src_slot >= 0) r.kind |= kRelSrcBuf;
     if (buf_dst && h.dst_slot >= 0) r.kind |= kRelDstBuf;
-    const uint32_t rec_bytes = record_bytes(h, tile_bytes);
+    const uint32_t rec_bytes = record_bytes(h, tile_bytes, few);
     r.kind |= log2u(rec_bytes) << kRelShiftBit;
     if (!h.contiguous && spans_far(h, rec_bytes)) r.kind |= kRelFar;
     r.src_slot = h.src_slot;
@@ -1316,7 +1320,7 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
     const uint64_t item_tile = uint64_t(tile_bytes) >> tile_reduce(h);
     ph.n_tiles += (r.total + item_tile - 1) / item_tile;
     const uint64_t recs = (r.total + rec_bytes - 1) / rec_bytes;
-    if (!h.contiguous && h.kind == kKindCopy) row_recs += recs;
+    if (!h.contiguous && h.kind == kKindCopy && h.row_bytes % 16 == 0 && h.row_bytes >= 512) row_recs += recs;
     ph.n_recs += recs;
     ph.rec_bytes += r.total;
   }
@@ -1344,7 +1348,7 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
       const HostItem& b = ph.items[order[i]];
       const Side sa = side(a), sb = side(b);
       chain = !a.contiguous && !b.contiguous && a.kind == b.kind && a.rows == b.rows &&
-              a.row_bytes == b.row_bytes && record_bytes(a, tile_bytes) == record_bytes(b, tile_bytes) && sa.slot >= 0 && sa.slot == sb.slot &&
+              a.row_bytes == b.row_bytes && record_bytes(a, tile_bytes, few) == record_bytes(b, tile_bytes, few) && sa.slot >= 0 && sa.slot == sb.slot &&
               sa.stride == sb.stride && sb.off == sa.off + sa.width;
     }
     if (!chain) {
