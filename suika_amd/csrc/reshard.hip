@@ -540,9 +540,8 @@ __device__ __forceinline__ void wide_tile(const DevItem& it, const DevTile& t, u
 // width apart: each vector's lines are then written by one wave (side by
 // side f32 rows of 16396 bytes: 5.7 TB/s, with the vectors of a lane a
 // workgroup's width apart 5.2).
-template <uint32_t KIND, int VB, Policy POLICY, bool NT, int B>
+template <uint32_t KIND, int VB, Policy POLICY, bool NT, int B, int W = VB == 8 ? 2 : 4>
 __device__ __forceinline__ void narrow_tile(const DevItem& it, const DevTile& t, uint32_t nbytes, const Ahead& ahead) {
-  constexpr int W = VB == 8 ? 2 : 4;
   constexpr uint32_t kStep = 64 * VB;
   const bool strided = it.row_bytes != 0;
   const Regions r = row_regions(it, strided ? t.src : 0);
@@ -669,7 +668,8 @@ __device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, co
         const DevItem it = items[t.item];
         rows_tile<kKindCopy, kStream, NT, B, U>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
       } else if (op == kOpRows8) {
-        narrow_tile<kKindCopy, 8, kStream, NT, B>(items[t.item], t, nbytes, ahead);
+        if (nbytes > B * 16) narrow_tile<kKindCopy, 8, kStream, NT, B, 4>(items[t.item], t, nbytes, ahead);
+        else narrow_tile<kKindCopy, 8, kStream, NT, B>(items[t.item], t, nbytes, ahead);
       } else if (op == kOpRows4) {
         narrow_tile<kKindCopy, 4, kStream, NT, B>(items[t.item], t, nbytes, ahead);
       } else if (op == kOpWide) {
@@ -738,19 +738,25 @@ constexpr uint32_t shape_lanes(Shape s) { return s == kSmall ? 512 : s == kTiny 
 constexpr uint64_t kFewTiles = 5120, kManyTiles = 16384;
 constexpr uint32_t kFewBlocks = 512;
 
-// The phase's tiles number more than a few, but not many, and are large.
-bool middling(uint64_t n_recs, uint64_t bytes) {
-  return n_recs > kFewTiles && n_recs <= kManyTiles && bytes / n_recs > 12 * 1024;
+// More bytes than kManyTiles whole tiles.
+bool large_phase(uint64_t bytes, uint32_t tile_bytes) { return bytes / tile_bytes > kManyTiles; }
+
+// The phase's tiles number more than a few, but not many, and are not small.
+bool middling(uint64_t n_recs, uint64_t bytes, uint32_t tile_bytes) {
+  return n_recs > kFewTiles && !large_phase(bytes, tile_bytes) && bytes / n_recs > 12 * 1024;
 }
 
-// `row_recs`: the tiles of COPY rows of 512 bytes and more and of a multiple of
-// 16 (of 16 bytes, 16384 tiles: 117 us with 1024 lanes, 132 with 512).
-Shape pick_shape(uint64_t n_recs, uint64_t bytes, uint64_t row_recs, uint32_t tile_bytes, uint32_t max_blocks) {
+// `rows`: the tiles of COPY rows of 512 bytes and more and of a multiple of 8
+// (of 16 bytes, 16384 tiles: 117 us with 1024 lanes, 132 with 512), and of
+// RECAST into bf16 alone (9000 tiles 43.2 / 38.3).  `recast`: those of RECAST
+// with an f32 copy, which count twice as few (4000 tiles 29.3 / 31.2).
+Shape pick_shape(uint64_t n_recs, uint64_t bytes, uint64_t rows, uint64_t recast, const sr_plan_options& opt) {
   const uint64_t mean = bytes / n_recs;
   if (mean <= 7 * 1024) return kTiny;
-  if (tile_bytes > kPassBytes) return kLong;
-  if (mean <= 12 * 1024 || n_recs <= kFewTiles || (max_blocks != 0 && max_blocks <= kFewBlocks)) return kSmall;
-  return middling(n_recs, bytes) && 2 * row_recs > n_recs ? kSmall : kWide;
+  if (opt.tile_bytes > kPassBytes) return kLong;
+  if (mean <= 12 * 1024 || n_recs + recast <= kFewTiles) return kSmall;
+  if (opt.max_blocks != 0 && opt.max_blocks <= kFewBlocks) return kSmall;
+  return middling(n_recs, bytes, opt.tile_bytes) && 2 * rows > n_recs ? kSmall : kWide;
 }
 
 // ------------------------------------------------- device-side plan binding
@@ -1228,12 +1234,20 @@ uint32_t tile_reduce(const HostItem& h) {
 // Source bytes of a tile record: what a workgroup moves in one pass, or
 // tile_bytes where that is more; for RECAST with an f32 copy the tile as plans
 // count it (16 MiB tiles of such rows: 911 us with twice as much, 692 so).
-// RECAST into bf16 alone moves 1.5 x its source bytes, and a tile of it too
-// little for its start: two passes, except in phases of `few` tiles (rows of
-// 16 KiB split off 139 us with one, 123 with two; merged 278 / 244; rows of
-// 2732 bytes merged 359 / 285).
-uint32_t record_bytes(const HostItem& h, uint32_t tile_bytes, bool few) {
-  if (h.kind == kKindRecast && h.dst_slot < 0 && tile_bytes <= kPassBytes && !few) return tile_bytes * 2;
+// In phases that are `large`, two passes for
+//   * RECAST into bf16 alone, which moves 1.5 x its source bytes, too little
+//     for a workgroup's start (rows of 16 KiB split off 139 us with one, 123
+//     with two; merged 278 / 244; rows of 2732 bytes merged 359 / 285);
+//   * COPY rows of 4 KiB and more that only 8-byte vectors divide (rows of
+//     16392 bytes split off 186 us with one, 177 with two; merged 183 / 181;
+//     of 1032 bytes merged 189 / 204).
+uint32_t record_bytes(const HostItem& h, uint32_t tile_bytes, bool large) {
+  if (large && tile_bytes <= kPassBytes) {
+    if (h.kind == kKindRecast && h.dst_slot < 0) return tile_bytes * 2;
+    if (h.kind == kKindCopy && !h.contiguous && h.row_bytes >= 4096 &&
+        ((h.row_bytes | h.src_stride | h.dst_stride) & 15) == 8)
+      return tile_bytes * 2;
+  }
   return std::max(tile_bytes >> tile_reduce(h), std::min(tile_bytes, kPassBytes));
 }
 
@@ -1250,8 +1264,8 @@ bool spans_far(const HostItem& h, uint32_t bytes) {
 // through 201).  Others written through are faster in large phases and in
 // those of few tiles (us, through / streamed: columns merged, 1500 tiles
 // 9.4 / 13.1, 40000 209 / 213; flat, 40000 tiles 200 / 203), but not
-//   * between, where much of the phase fits the memory-side cache, for rows
-//     and RECAST (columns merged, 6000 tiles 36.5 / 35.7, 9000 53.2 / 51.6,
+//   * between, where much of the phase fits the memory-side cache, for RECAST
+//     and rows of 512 bytes and more (columns merged, 6000 tiles 36.5 / 35.7, 9000 53.2 / 51.6,
 //     20000 108.7 / 108.8; RECAST, merged, 6000 tiles 46.2 / 43.2, 40000
 //     264.8 / 267.1);
 //   * into rows that the launch does not write side by side from end to end
@@ -1261,12 +1275,12 @@ bool spans_far(const HostItem& h, uint32_t bytes) {
 //     (1 GiB, 64 workgroups 1026 / 934, 1 MiB tiles 405 / 400).
 bool stream_whole(const HostItem& h, uint32_t group_size, const Phase& ph, const sr_plan_options& opt) {
   if (h.kind == kKindZero) return !h.contiguous;
-  if (h.kind == kKindRecast) return h.dst_slot >= 0 && middling(ph.n_recs, ph.rec_bytes);
+  if (h.kind == kKindRecast) return middling(ph.n_recs, ph.rec_bytes, opt.tile_bytes);
   const bool loops = opt.tile_bytes > kPassBytes || (opt.max_blocks != 0 && opt.max_blocks <= kFewBlocks);
   if (h.contiguous && loops) return true;
   if (h.contiguous || ph.n_recs <= kFewTiles) return false;
   const bool side_by_side = h.dst_stride == h.row_bytes || h.dst_stride == h.row_bytes * group_size;
-  return !side_by_side || middling(ph.n_recs, ph.rec_bytes);
+  return !side_by_side || (h.row_bytes >= 512 && middling(ph.n_recs, ph.rec_bytes, opt.tile_bytes));
 }
 
 void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_options& opt, bool buf_src,
@@ -1278,9 +1292,9 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
   ph.tile_base.clear();
   ph.tile_base.reserve(order.size() + 1);
   ph.n_tiles = ph.n_recs = ph.rec_bytes = 0;
-  uint64_t row_recs = 0, all_bytes = 0;
+  uint64_t row_recs = 0, recast_recs = 0, all_bytes = 0;
   for (const HostItem& h : ph.items) all_bytes += h.rows * h.row_bytes;
-  const bool few = all_bytes / tile_bytes <= kFewTiles;
+  const bool large = large_phase(all_bytes, tile_bytes);
   for (uint32_t k : order) {
     ph.tile_base.push_back(ph.n_recs);
     const HostItem& h = ph.items[k];
@@ -1303,7 +1317,7 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
     r.kind = h.kind | (h.esize << 8);
     if (buf_src && h.src_slot >= 0) r.kind |= kRelSrcBuf;
     if (buf_dst && h.dst_slot >= 0) r.kind |= kRelDstBuf;
-    const uint32_t rec_bytes = record_bytes(h, tile_bytes, few);
+    const uint32_t rec_bytes = record_bytes(h, tile_bytes, large);
     r.kind |= log2u(rec_bytes) << kRelShiftBit;
     if (!h.contiguous && spans_far(h, rec_bytes)) r.kind |= kRelFar;
     r.src_slot = h.src_slot;
@@ -1320,12 +1334,15 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
     const uint64_t item_tile = uint64_t(tile_bytes) >> tile_reduce(h);
     ph.n_tiles += (r.total + item_tile - 1) / item_tile;
     const uint64_t recs = (r.total + rec_bytes - 1) / rec_bytes;
-    if (!h.contiguous && h.kind == kKindCopy && h.row_bytes % 16 == 0 && h.row_bytes >= 512) row_recs += recs;
+    const bool half_only = h.kind == kKindRecast && h.dst_slot < 0;
+    const bool rows = !h.contiguous && h.kind == kKindCopy && h.row_bytes % 8 == 0 && h.row_bytes >= 512;
+    if (half_only || rows) row_recs += recs;
+    else if (h.kind == kKindRecast) recast_recs += recs;
     ph.n_recs += recs;
     ph.rec_bytes += r.total;
   }
   ph.tile_base.push_back(ph.n_recs);
-  if (ph.n_recs > 0) ph.shape = pick_shape(ph.n_recs, ph.rec_bytes, row_recs, tile_bytes, opt.max_blocks);
+  if (ph.n_recs > 0) ph.shape = pick_shape(ph.n_recs, ph.rec_bytes, row_recs, recast_recs, opt);
   ph.emit_chunks.clear();
   for (size_t k = 0; k < ph.rel.size(); ++k) {
     const uint64_t cnt = ph.tile_base[k + 1] - ph.tile_base[k];
@@ -1348,7 +1365,7 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
       const HostItem& b = ph.items[order[i]];
       const Side sa = side(a), sb = side(b);
       chain = !a.contiguous && !b.contiguous && a.kind == b.kind && a.rows == b.rows &&
-              a.row_bytes == b.row_bytes && record_bytes(a, tile_bytes, few) == record_bytes(b, tile_bytes, few) && sa.slot >= 0 && sa.slot == sb.slot &&
+              a.row_bytes == b.row_bytes && record_bytes(a, tile_bytes, large) == record_bytes(b, tile_bytes, large) && sa.slot >= 0 && sa.slot == sb.slot &&
               sa.stride == sb.stride && sb.off == sa.off + sa.width;
     }
     if (!chain) {

@@ -195,6 +195,28 @@ def test_streamed_lines(rows, tile_bytes):
     e.check(flat.t, "whole rows")
 
 
+@pytest.mark.parametrize("rows,tile_bytes", [(19000, 4096), (66000, 0), (5000, 0)])
+@pytest.mark.parametrize("cols", [1026, 1025, 1032, 33])
+def test_two_pass_records(cols, rows, tile_bytes):
+    """Bands in large phases, where rows in 8-byte vectors and RECAST into bf16
+    alone have records of two passes, and in a small one: split, merged, and
+    rounded, side by side with pieces of one pass."""
+    print(f"[copy forms] bands of {cols}, {rows} rows, tile {tile_bytes}", flush=True)
+    rows = rows * (31 if cols == 33 else 1)
+    w = Obj(rows, 2 * cols, "f32", seed=cols)
+    x, h, d, f = Obj(rows, cols, "f32"), Obj(rows, cols, "bf16"), Obj(rows, 2 * cols, "bf16"), Obj(rows, cols, "f32")
+    _gather([w], [x, h, f], [copy(0, 0, rows, cols, sc=cols), (RECAST, 0, 0, -1, 1, 0, rows, cols, 0, 0, 0, 0),
+                             copy(0, 2, rows, cols)], tile_bytes)
+    x.check(w.t[:, cols:], "split")
+    h.check(w.t[:, :cols].to(torch.bfloat16), "rounded")
+    e = Obj(rows, 2 * cols, "f32")
+    _gather([x, f], [d, e], [(RECAST, 0, 1, -1, 0, 0, rows, cols, 0, 0, 0, 0),
+                             (RECAST, 0, 0, -1, 0, 0, rows, cols, 0, 0, 0, cols), copy(1, 1, rows, cols),
+                             copy(0, 1, rows, cols, dc=cols)], tile_bytes)
+    d.check(w.t.to(torch.bfloat16), "merged, rounded")
+    e.check(w.t, "merged")
+
+
 def test_rows_two_gib_apart():
     """Rows so long that a tile's rows span 2 GiB: 64-bit offsets, beside a
     band of the same rows that is near enough within a smaller tile."""
