@@ -175,3 +175,90 @@ def test_graph_capture_stays_refused():
         assert torch.equal(mark, torch.full_like(mark, 4.0))
     finally:
         p.close()
+
+
+def test_first_use_in_a_capture():
+    """A small phase whose first use is captured has tables that the graph's
+    launches build on the device: each replay gives the bytes of the sources
+    as they then are, with other plans' launches and host waits between."""
+    print("[gpu host tables] first use captured", flush=True)
+    p, q, other = Plan(64), Plan(64), Plan(64)
+    src, dst, back = p.src(0), p.dst(), p.dst()
+    buf = torch.empty(q.peer_bytes, dtype=torch.uint8, device="cuda")
+    new = [p.src(i) for i in (1, 2, 3)]
+    busy = p.dst()
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    try:
+        with torch.cuda.stream(stream):
+            with torch.cuda.graph(g, stream=stream, capture_error_mode="relaxed"):
+                p.gather(src, dst)
+                q.exchange(src, buf, back)
+            for fresh in new:
+                for a, b in zip(src, fresh):
+                    a.copy_(b)
+                for t in dst + back:
+                    t.fill_(7)
+                buf.fill_(0xA5)
+                g.replay()
+                other.gather(fresh, busy)
+                torch.cuda.synchronize()
+                p.check(fresh, dst)
+                p.check(fresh, back)
+                other.check(fresh, busy)
+    finally:
+        torch.cuda.synchronize()
+        del g
+        for plan in (p, q, other):
+            plan.close()
+
+
+@pytest.mark.parametrize("cols", [512, 513, 514, 516])
+@pytest.mark.parametrize("rows", [700, 5000])
+def test_device_tables_rebound(rows, cols):
+    """Above the limit, in phases of a few and of many thousand tiles: columns
+    put together, and the same rounded, in row groups, and zero-filled rows,
+    with bindings taking turns and no host wait."""
+    parts, zeros = 3, 2
+    print(f"[gpu host tables] {parts} x [{rows}, {cols}] put together, pointers in turn", flush=True)
+    L, T, piece = _lib.lib(), _lib.SrTensor, _lib.SrPiece
+    f32, bf16 = _lib.SR_DT_F32, _lib.SR_DT_BF16
+    S = (T * parts)(*[T(rows, cols, f32, 0)] * parts)
+    D = (T * 2)(T(rows + zeros, parts * cols, f32, 0), T(rows, parts * cols, bf16, 0))
+    P = [piece(_lib.SR_PIECE_COPY, 0, k, 0, -1, 0, rows, cols, 0, 0, 0, k * cols) for k in range(parts)]
+    P += [piece(_lib.SR_PIECE_RECAST, 0, k, -1, 1, 0, rows, cols, 0, 0, 0, k * cols) for k in range(parts)]
+    P.append(piece(_lib.SR_PIECE_ZERO, 0, -1, 0, -1, 0, zeros, parts * cols, 0, 0, rows, 0))
+    h, n = vp(), ctypes.c_uint64()
+    _lib.check(L.sr_plan_create(S, parts, D, 2, 1, (piece * len(P))(*P), len(P),
+                                ctypes.byref(_lib.SrPlanOptions(TILE, 0, 0, 0)), ctypes.byref(h)), "plan")
+
+    def call(fn, a, b):
+        A, B = (vp * len(a))(*[t.data_ptr() for t in a]), (vp * len(b))(*[t.data_ptr() for t in b])
+        _lib.check(fn(h, A, B, vp(torch.cuda.current_stream().cuda_stream)), "call")
+
+    try:
+        _lib.check(L.sr_plan_peer_bytes(h, 0, ctypes.byref(n)), "peer bytes")
+        assert 2 * parts * rows * cols * 4 // TILE > LIMIT
+        g = torch.Generator("cuda").manual_seed(cols)
+        srcs = [[torch.randn(rows, cols, generator=g, device="cuda") for _ in range(parts)] for _ in range(3)]
+        dsts = [[torch.empty(rows + zeros, parts * cols, device="cuda"),
+                 torch.empty(rows, parts * cols, device="cuda", dtype=torch.bfloat16)] for _ in range(3)]
+        bufs = [torch.empty(n.value, dtype=torch.uint8, device="cuda") for _ in range(3)]
+        for route in ("gather", "exchange"):
+            for i in (0, 1, 2, 1, 1, 0, 2, 2, 0):
+                for t in dsts[i]:
+                    t.fill_(7)
+                if route == "gather":
+                    call(L.sr_gather, srcs[i], dsts[i])
+                else:
+                    bufs[i].fill_(0xA5)
+                    call(L.sr_pack, srcs[i], [bufs[i]])
+                    call(L.sr_unpack, [bufs[i]], dsts[i])
+            for i, (s, d) in enumerate(zip(srcs, dsts)):
+                want = torch.cat(s, 1)
+                assert torch.equal(d[0], torch.cat([want, want.new_zeros(zeros, parts * cols)])), (route, i, "copy")
+                assert torch.equal(d[1], want.to(torch.bfloat16)), (route, i, "rounded")
+    finally:
+        torch.cuda.synchronize()
+        L.sr_plan_destroy(h)
