@@ -119,7 +119,8 @@ typedef struct sr_plan_options {
                             this size */
   uint32_t max_blocks;   /* cap on workgroups per launch (grid-stride beyond;
                             rounded down to a multiple of 8 when the tile list
-                            is XCD-interleaved); 0 = one workgroup per tile */
+                            is XCD-interleaved); 0 = one workgroup per tile,
+                            or per two tiles of a kind that is faster so */
   uint32_t flags;        /* SR_OPT_* bits */
   uint32_t reserved;     /* must be 0 */
 } sr_plan_options;

@@ -19,19 +19,21 @@
 //   * Items are cut into tiles of `tile_bytes` (16 KiB) source bytes; one
 //     workgroup (1024 lanes = 16 wave64) moves one tile, 16 bytes per lane,
 //     and the grid is the tile count (or a grid-stride loop when capped).
-//     Phases of few, small or several-pass tiles have other workgroups (Shape).
+//     Phases of few, small or several-pass tiles have other workgroups (Shape),
+//     and some items of large phases two tiles to a workgroup (record_bytes).
 //     Tiles balance the work whatever the tensor sizes (8 KB norms to GB
 //     embeddings).
 //   * A lane loads once, stores once and ends.  Two workgroups fill a compute
-//     unit, so 32 KiB of reads are in flight there: HBM moves a flat copy at
-//     6.7 TB/s with that, at 6.2 with twice as much (two loads per lane), and
-//     at 4.1-5.4 with waves that go on to another tile, because a load's data
-//     is waited for behind the stores issued before it.
+//     unit, so 32 KiB of reads are in flight there: HBM moves a flat copy of
+//     2 GiB at 6.65 TB/s with that, at 6.1 with twice as much (two loads per
+//     lane of 512), and at 4.1-5.4 with waves that go on to another tile,
+//     because a load's data is waited for behind the stores issued before it.
 //   * So the way from the launch to the load is short: the kernel arguments
 //     arrive in registers, a tile's record holds the addresses of a
 //     contiguous copy, a record line is read into the die's L2 256 tiles
-//     before its workgroup starts (without that: 6.4 TB/s), and the forms of
-//     large tensors come first in a kernel of 20 KB (46 KB: 3% slower).
+//     before its workgroup starts, the lines of the next items with it
+//     (Ahead), and the forms of large tensors come first in a kernel of 26 KB
+//     (one of 46 KB, before the forms were folded: 3% slower).
 //   * The tile list follows the tensor address each item starts at and is cut
 //     into 8 segments: workgroups go to the 8 XCDs round-robin, so each XCD
 //     walks one contiguous eighth of the list (and of its records) and the
@@ -61,18 +63,21 @@
 //   * sr_plan_create is host only and O(pieces): validation, coverage, the
 //     buffer layout the API reports, and one pointer-independent descriptor
 //     per item.  The CPU test-suite exercises it without a GPU.
-//   * The O(tiles) work runs on the GPU at first use of a phase: prefix sums
-//     (wave64 shuffle scans, wave totals through LDS) give each peer's
-//     256-byte aligned buffer offsets and each item's first tile, and an emit
-//     kernel writes the tile table.  The
-//     Llama2-7B share has 1.44 M tiles per phase; building them on the host
-//     took 0.12 s and a 35 MB upload per phase.
-//   * Tile records and items hold absolute addresses.  When the caller's
-//     pointers change, only the pointer table is uploaded and the emit kernel
-//     writes both again from the descriptors and the device-side buffer
-//     offsets.  (Read in place in pinned memory, without the upload, the emit
-//     is 1 us a launch slower: 4096 tiles 33.1 -> 34.1 us.)
-//   * Phases of few tiles have their tables written by the host (run_small).
+//     Each item's first tile is a prefix sum over the items.
+//   * Phases of at most kHostTableTiles tiles have their tables written by the
+//     host, at each launch on new pointers (run_small).
+//   * The O(tiles) work of larger ones runs on the GPU at first use of a
+//     phase: an emit kernel writes the tile table, and prefix sums (wave64
+//     shuffle scans, wave totals through LDS) give each peer's 256-byte
+//     aligned buffer offsets.  The Llama2-7B share has 1.44 M tiles per phase;
+//     building them on the host took 0.12 s and a 35 MB upload per phase.
+//   * Tile records and items hold absolute addresses.  When the pointers of a
+//     larger phase change, only the pointer table is uploaded and the emit
+//     kernel writes both again from the descriptors and the device-side buffer
+//     offsets (2624 to 16384 tiles 4.1-4.4 us; a table of items alone, bound
+//     by a kernel of one lane per item, took 4.2).  Read in place in pinned
+//     memory, without the upload, the emit is 1 us a launch slower (4096 tiles
+//     33.1 -> 34.1 us).
 
 #include <hip/hip_runtime.h>
 
@@ -268,8 +273,8 @@ constexpr uint32_t kNowhere = 0xfffffff0u;
 // Cache policies: the aux bits of gfx950's buffer instructions (2 = nt,
 // 16 = sc1).  Loads are non-temporal.  Stores of whole 64-byte lines write
 // through the L2: the lines then do not wait there for an eviction that
-// competes with the reads (flat copy of 2 GiB: 6.8 TB/s, nt 6.55; zero fill
-// 7.5, nt 6.5).  Lines that several waves or rows write in parts are left for
+// competes with the reads (flat copy of 2 GiB: 6.65 TB/s, nt 6.50; zero fill
+// of 4 GiB 7.66, nt 6.90).  Lines that several waves or rows write in parts are left for
 // the L2 to merge, as streaming lines or, for short rows, as ordinary ones
 // (side by side rows of 4 bytes: through 3.0 TB/s, nt 3.6, ordinary 5.1; of
 // 36 kB + 16 bytes: 5.4, 5.9, 5.5).  Where whole lines are streamed all the
@@ -428,8 +433,8 @@ __device__ __forceinline__ void put(const Regions& r, const Place& at, typename 
 // line), so that a record is there when its workgroup starts.  The read is
 // issued behind the tile's loads and done with before its stores: a wait
 // after them would hold the wave until they are written.  256 records cover a
-// die's tiles in flight twice over (flat copy of 2 GiB: 6.40 TB/s without,
-// 6.69 with 256 or 512 ahead, 6.47 with 2048).
+// die's tiles in flight twice over (flat copy of 2 GiB: 6.26 TB/s without,
+// 6.65 with; 512 ahead gave the same, 2048 3% less).
 //
 // The same read takes the lines of the next 16 items along, for tiles that
 // need theirs: each new item's line otherwise stops all the tiles that are in
@@ -668,7 +673,8 @@ __device__ __forceinline__ void exec_tiles(const DevItem* __restrict__ items, co
         const DevItem it = items[t.item];
         rows_tile<kKindCopy, kStream, NT, B, U>(row_regions(it, t.src), it, uint32_t(t.dst), nbytes, ahead);
       } else if (op == kOpRows8) {
-        if (nbytes > B * 16) narrow_tile<kKindCopy, 8, kStream, NT, B, 4>(items[t.item], t, nbytes, ahead);
+        // a body of four vectors in the workgroups of large phases too costs their merged rows 1%
+        if (U == 2 && nbytes > B * 16) narrow_tile<kKindCopy, 8, kStream, NT, B, 2 * U>(items[t.item], t, nbytes, ahead);
         else narrow_tile<kKindCopy, 8, kStream, NT, B>(items[t.item], t, nbytes, ahead);
       } else if (op == kOpRows4) {
         narrow_tile<kKindCopy, 4, kStream, NT, B>(items[t.item], t, nbytes, ahead);
@@ -727,8 +733,8 @@ SR_COPY_KERNEL(sr_gather_kernel)
 //     24.5 / 21.7, 6000 36.5 / 36.5), and up to 16384 where most are COPY
 //     rows, which then are streamed (1024 lanes of one / 512 of two: 8192
 //     tiles 50.8 / 49.1, 16384 91.8 / 89.1; contiguous ones 46.9 / 48.8);
-//   * grids capped at 512 workgroups or less, the same (1 GiB, 64 workgroups
-//     1123 / 1026 us, 256 421 / 378, 512 394 / 388);
+//   * grids capped at 512 workgroups or less, the same (1 GiB of columns
+//     merged, 64 workgroups 1198 / 1000 us, 256 405 / 370, 512 448 / 421);
 //   * tiles of more than one pass: two vectors in each of 1024 lanes (64 KiB
 //     tiles, columns merged 381 / 356 us with one / two).
 enum Shape { kWide, kSmall, kTiny, kLong };
@@ -746,8 +752,10 @@ bool middling(uint64_t n_recs, uint64_t bytes, uint32_t tile_bytes) {
   return n_recs > kFewTiles && !large_phase(bytes, tile_bytes) && bytes / n_recs > 12 * 1024;
 }
 
-// `rows`: the tiles of COPY rows of 512 bytes and more and of a multiple of 8
-// (of 16 bytes, 16384 tiles: 117 us with 1024 lanes, 132 with 512), and of
+// `rows`: the tiles of COPY rows of 512 bytes and more and of a multiple of 16
+// (of 16 bytes, 16384 tiles: 117 us with 1024 lanes, 132 with 512), or of 8
+// where they are written end to end (9000 tiles, rows of 4104 bytes split off
+// 55.6 / 53.2, but merged 56.4 / 56.7, of 1032 merged 57.7 / 61.4), and of
 // RECAST into bf16 alone (9000 tiles 43.2 / 38.3).  `recast`: those of RECAST
 // with an f32 copy, which count twice as few (4000 tiles 29.3 / 31.2).
 Shape pick_shape(uint64_t n_recs, uint64_t bytes, uint64_t rows, uint64_t recast, const sr_plan_options& opt) {
@@ -761,8 +769,9 @@ Shape pick_shape(uint64_t n_recs, uint64_t bytes, uint64_t rows, uint64_t recast
 
 // ------------------------------------------------- device-side plan binding
 // The host keeps O(pieces) descriptors and the prefix sum of their tile
-// counts; the per-tile table, the per-peer buffer offsets and the
-// absolute-address item table are computed on the GPU from them:
+// counts; for phases above kHostTableTiles the per-tile table, the per-peer
+// buffer offsets and the absolute-address item table are computed on the GPU
+// from them:
 //   sr_offsets_kernel   per peer: exclusive prefix sum of the 256-byte
 //                       rounded payloads of its pieces, in piece order;
 //   sr_tile_emit_kernel one workgroup per chunk of an item's tiles writes
@@ -1238,13 +1247,14 @@ uint32_t tile_reduce(const HostItem& h) {
 //   * RECAST into bf16 alone, which moves 1.5 x its source bytes, too little
 //     for a workgroup's start (rows of 16 KiB split off 139 us with one, 123
 //     with two; merged 278 / 244; rows of 2732 bytes merged 359 / 285);
-//   * COPY rows of 4 KiB and more that only 8-byte vectors divide (rows of
-//     16392 bytes split off 186 us with one, 177 with two; merged 183 / 181;
-//     of 1032 bytes merged 189 / 204).
+//   * COPY rows that only 8-byte vectors divide, of 4 KiB and more written end
+//     to end (1 GiB of rows of 4104 bytes split off 375 us with one, 369 with
+//     two; of 1032 bytes 385 / 413) and of 16 KiB and more otherwise (of
+//     4104 bytes merged 368 / 374, of 32776 bytes 366 / 355).
 uint32_t record_bytes(const HostItem& h, uint32_t tile_bytes, bool large) {
   if (large && tile_bytes <= kPassBytes) {
     if (h.kind == kKindRecast && h.dst_slot < 0) return tile_bytes * 2;
-    if (h.kind == kKindCopy && !h.contiguous && h.row_bytes >= 4096 &&
+    if (h.kind == kKindCopy && !h.contiguous && h.row_bytes >= (h.dst_stride == h.row_bytes ? 4096 : 16384) &&
         ((h.row_bytes | h.src_stride | h.dst_stride) & 15) == 8)
       return tile_bytes * 2;
   }
@@ -1335,7 +1345,8 @@ void build_rel(Phase& ph, const std::vector<uint32_t>& order, const sr_plan_opti
     ph.n_tiles += (r.total + item_tile - 1) / item_tile;
     const uint64_t recs = (r.total + rec_bytes - 1) / rec_bytes;
     const bool half_only = h.kind == kKindRecast && h.dst_slot < 0;
-    const bool rows = !h.contiguous && h.kind == kKindCopy && h.row_bytes % 8 == 0 && h.row_bytes >= 512;
+    const bool rows = !h.contiguous && h.kind == kKindCopy && h.row_bytes >= 512 &&
+                      h.row_bytes % (h.dst_stride == h.row_bytes ? 8 : 16) == 0;
     if (half_only || rows) row_recs += recs;
     else if (h.kind == kKindRecast) recast_recs += recs;
     ph.n_recs += recs;
