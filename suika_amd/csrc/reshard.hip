@@ -1835,15 +1835,14 @@ int run_phase(sr_plan* p, Phase& ph, PhaseKind kind, const std::vector<uint64_t>
     if (rc != SR_OK) return rc;
     if (setup != stream) SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_setup, 0));
   } else if (rebind) {
-    // Later rebinds run on `stream`, after the latest bind (whose copy out
-    // of the staging buffer must be done before the host rewrites it) and
-    // after the phase's previous launch (which may still read the item and
-    // pointer tables).
+    // Later rebinds run on `stream`.  The latest bind's copy out of the
+    // staging buffer must be done before the host rewrites it, and the bind
+    // follows the phase's previous launch, which may still read the tables
+    // (and followed the bind before it: one wait for both).
     if (!ph.ev_staging && (rc = table_cache().get_event(p->device, &ph.ev_staging)) != SR_OK) return rc;
     SR_HIP_TRY(hipEventSynchronize(ph.ev_bound));
     std::memcpy(ph.h_ptrs, ptrs.data(), ptrs.size() * sizeof(uint64_t));
-    SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_bound, 0));
-    SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_kernel, 0));
+    SR_HIP_TRY(hipStreamWaitEvent(stream, ph.ev_tail, 0));
     SR_HIP_TRY(hipMemcpyAsync(ph.d_ptrs, ph.h_ptrs, ptrs.size() * sizeof(uint64_t), hipMemcpyHostToDevice,
                               stream));
     if ((rc = emit_tables(p, ph, stream)) != SR_OK) return rc;
